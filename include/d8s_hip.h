@@ -248,6 +248,13 @@ int d8s_dense_block(const D8sBlockArgs* a, void* stream);
 int d8s_dense_block_parts(const D8sPartsArgs* a, void* stream);
 int d8s_parts_supported(int32_t H, int32_t W, int32_t G, int32_t parts);
 
+/* d8s_dense_block_parts for maps whose rows make no whole 32-pixel tiles (72, 36, 18 and 9 wide at 288
+ * px): `parts` bands of H / parts rows, the first H % parts of them one row more, at most 256 pixels
+ * each; the same bytes, and the same sync and xchg memory, waits and final check as
+ * d8s_dense_block_parts.  d8s_bands_supported(H, W, G0 + L - 1, parts) says whether a shape is taken. */
+int d8s_dense_block_bands(const D8sPartsArgs* a, void* stream);
+int d8s_bands_supported(int32_t H, int32_t W, int32_t G, int32_t bands);
+
 /* Transition: prologue on the 4 pixels of every 2x2 square, s = sum of the four u, S = sum_k w[o][k]
  * s[k] (exact int32), q = RNE(clamp(k'_o * (float(S) / 4), -127, 127)) into the next block's in0.
  * H and W even, cout a multiple of 32 (at most 1024), N * HW < 2^31 and the in0 / one seg slot below

@@ -20,6 +20,7 @@
 #include <string.h>
 
 #include <algorithm>
+#include <atomic>
 #include <string>
 #include <type_traits>
 
@@ -2164,9 +2165,23 @@ __global__ __launch_bounds__(DB_NT, 1) void k_dblock(D8sBlockArgs a0, D8sBlockAr
 // last workgroup to end resets the ticket and the end count and advances the launch count (sync[3])
 // the tags are made of, so the next launch needs no clearing.  Tables, weights and the next pass's
 // first chunk of store bytes are requested a phase ahead of their use.
+// What bounds it: each layer's chain of phases (set-up, conv1 loop, exchange, conv2, epilogue: 2.2, 5.7,
+// 3.0, 2.8 and 2.4 thousand cycles for the 16 x 16 block's 32-pixel bands, of which 1.3 of the exchange now
+// run beside the loop), so a launch takes as long as a layer's chain times the layers whatever the
+// band count that fits the CUs; within the loop each CU streams every layer's weights itself.  Three
+// things took the two blocks of a 24-image study (8 bands) from 341 + 239 to 319 + 210 us, 4 bands of
+// the 32 x 32 block from 554 to 457 us: loads past a layer's last group read nothing (buffer loads out
+// of range) where they had read the last group again, a wave's prologue items of a chunk share one
+// group's table, and the neighbours' rows are requested before the loop's last chunk.
 // ------------------------------------------------------------------------------------------------
 static constexpr int DP_NT = 512;
 static constexpr int DP_SPIN = 1 << 20;                   // polls before a wait gives up
+static constexpr uint32_t DP_OOB = 0x40000000u;           // past any layer's weights
+// a wave-uniform 64-bit value read from LDS, in scalar registers
+DEV uint64_t uniform64(uint64_t v) {
+    return (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(v >> 32)) << 32 |
+           (uint32_t)__builtin_amdgcn_readfirstlane((int)v);
+}
 
 DEV uint64_t ld_agent64(const uint64_t* p) {
     return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -2180,13 +2195,13 @@ DEV void st_agent(uint32_t* p, uint32_t v) { __hip_atomic_store(p, v, __ATOMIC_R
 // Shape constants of k_dparts<PT>, shared by the kernel's static LDS arrays and the host's LDS check.
 template <int PT>
 struct DpShape {
-    static_assert(PT == 1 || PT == 2 || PT == 4 || PT == 8, "pixel tiles per band");
+    static_assert(PT == 1 || PT == 2 || PT == 4 || PT == 6 || PT == 8, "pixel tiles per band");
     // groups per prologue chunk: 4 for 128- and 256-pixel bands (for 128: a 24-image study's 32 x 32
     // block 0.76-0.77 against 0.79-0.82 ms with 8, 0.78-0.80 with 2), 8 for the narrower ones (a
     // 32-pixel band needs 8 for one operand per wave; 16 was slower)
-    static constexpr int CG = PT == 4 || PT == 8 ? 4 : 8;
+    static constexpr int CG = PT >= 4 ? 4 : 8;
     static constexpr int ITEMS = CG * PT;                  // (group, pixel tile) operands per chunk
-    static constexpr int S2 = PT == 8 ? 1 : (PT == 4 ? 2 : 4);   // conv2 K slices per pixel tile
+    static constexpr int S2 = PT >= 6 ? 1 : (PT == 4 ? 2 : 4);   // conv2 K slices per pixel tile
     static constexpr int NRED = PT == 1 ? 4 * 1024 : ((S2 - 1) * PT * 1024 > 0 ? (S2 - 1) * PT * 1024 : 1);
     static constexpr int NLP = 64 * 7;                     // layer descriptors (at most 64 layers)
     // static LDS bytes: conv2 weights, two prologue chunks, partial sums, the ticket words and the
@@ -2194,7 +2209,11 @@ struct DpShape {
     static constexpr size_t STATIC = 2304 * 16 + 2 * ITEMS * 64 * 16 + NRED * 4 + 2 * 4 + NLP * 8 + 64;
 };
 
-template <int PT>
+// RAG: bands of any row count and map width (d8s_dense_block_bands): band p has H / K rows, one more
+// for the first H % K bands, and its last pixel tiles may be partly or wholly past its pixels (those
+// lanes read the band's last pixel and store nothing).  The full-tile instances compile without the
+// masks: their bands are what d8s_dense_block_parts takes.
+template <int PT, bool RAG>
 __global__ __launch_bounds__(DP_NT, 1) void k_dparts(D8sPartsArgs a) {
     using SH = DpShape<PT>;
     constexpr int CG = SH::CG;
@@ -2203,10 +2222,10 @@ __global__ __launch_bounds__(DP_NT, 1) void k_dparts(D8sPartsArgs a) {
     constexpr int NPT = PT == 1 ? 1 : PT / 2;              // conv1 pixel tiles per wave
     constexpr int KH = PT == 1 ? 2 : 1;                    // conv1 K halves (32-pixel bands)
     constexpr int QC = CG / KH;                            // a wave's groups per chunk
-    constexpr int DW = 4;                                  // weight groups in flight per wave
+    constexpr int DW = QC;                                 // weight groups in flight per wave: a chunk's
     constexpr int S2 = SH::S2;                             // conv2 K slices per pixel tile
     constexpr int NRED = SH::NRED;
-    static_assert(QC % DW == 0 && IPW >= 1, "chunk shape");
+    static_assert(IPW >= 1 && 8 / CG * IPW == PT, "chunk shape");
     __shared__ __attribute__((aligned(16))) u32x4 s_w[2304];              // conv2 weights, 36 KB
     __shared__ __attribute__((aligned(16))) u32x4 s_pro[2 * ITEMS * 64];  // prologue chunks
     __shared__ __attribute__((aligned(16))) int32_t s_red[NRED];          // partial sums
@@ -2216,7 +2235,8 @@ __global__ __launch_bounds__(DP_NT, 1) void k_dparts(D8sPartsArgs a) {
     __shared__ uint64_t s_lp[SH::NLP];
     static_assert(sizeof(D8sLayerP) == 7 * sizeof(uint64_t), "descriptor layout");
     extern __shared__ __attribute__((aligned(16))) u32x4 s_dyn[];
-    const int H = a.H, W = a.W, HW = H * W, K = a.parts, R = H / K, BW = W + 2, WIN = (R + 2) * BW;
+    const int H = a.H, W = a.W, HW = H * W, K = a.parts, BW = W + 2;
+    const int RMAX = RAG ? (H + K - 1) / K : H / K, WIN = (RMAX + 2) * BW;
     const int G0 = a.G0, L = a.L, N = a.N;
     u32x4* s_b = s_dyn;                                                    // [4][WIN][2]
     int32_t* s_w1sum = (int32_t*)(s_dyn + 8 * WIN);                       // [128]
@@ -2246,6 +2266,10 @@ __global__ __launch_bounds__(DP_NT, 1) void k_dparts(D8sPartsArgs a) {
     const uint32_t epoch = s_tk[1];
     const int n = ticket / K, part = ticket - n * K;
     if (!valid && tid == 0) atomicAdd(sync + 2, 1u);
+    // the band's rows and first row
+    const int R = RAG ? H / K + (part < H % K ? 1 : 0) : RMAX;
+    const int r0 = RAG ? part * (H / K) + min(part, H % K) : part * R;
+    const int P = R * W;
     {
         const u32x4 pad = {SIGN4, SIGN4, SIGN4, SIGN4};
         for (int idx = tid; idx < WIN * 8; idx += DP_NT) {
@@ -2255,15 +2279,23 @@ __global__ __launch_bounds__(DP_NT, 1) void k_dparts(D8sPartsArgs a) {
                 s_b[cc * WIN * 2 + swz(wp, hh)] = pad;
         }
     }
-    const int bandp = part * R * W;                        // the band's first pixel in the image
+    const int bandp = r0 * W;                              // the band's first pixel in the image
     const uint8_t* img0 = (const uint8_t*)a.in0 + (int64_t)n * G0 * HW * 32;
     uint8_t* segn = (uint8_t*)a.seg + (int64_t)n * HW * 32;
     const int64_t slot = (int64_t)N * HW * 32;
     uint64_t* xpair = (uint64_t*)a.xchg;                  // [nparts][parity][top, bottom][4][W][8]
     bool broken = false;                                   // a wait ran out: skip the later ones
-    // store bytes of group g at band pixel 32 t + j (a uniform base plus the lane's 32-bit offset)
-#define DP_SRC(g, t) (((g) < G0 ? img0 + (int64_t)(g) * HW * 32 : segn + (int64_t)((g) - G0) * slot) + \
-                      (uint32_t)((bandp + 32 * (t) + j) * 32 + 16 * h))
+    // store bytes of group g at band pixel 32 t + j, t the pixel tile of a wave's item q (a uniform
+    // base plus the lane's 32-bit offset, kept per item where the band is ragged).  A wave's items are
+    // one group's (pg of the chunk's) for the pixel tiles pt0, pt0 + 1, ..: one read of its prologue table
+    const int pg = wave % CG, pt0 = wave / CG * IPW;
+    uint32_t ro[RAG ? IPW : 1];
+    if constexpr (RAG) {
+#pragma unroll
+        for (int q = 0; q < IPW; ++q) ro[q] = (bandp + min(32 * (pt0 + q) + j, P - 1)) * 32 + 16 * h;
+    }
+#define DP_GRP(g) ((g) < G0 ? img0 + (int64_t)(g) * HW * 32 : segn + (int64_t)((g) - G0) * slot)
+#define DP_OFF(q) (RAG ? ro[RAG ? (q) : 0] : (uint32_t)((bandp + 32 * (pt0 + (q)) + j) * 32 + 16 * h))
 #define DP_XP(tk, par, which, cc) (xpair + ((((int64_t)(tk) * 2 + (par)) * 2 + (which)) * 4 + (cc)) * W * 8)
     // a wave's conv1 groups: q -> g = q (PT >= 2) or 2 q + hv (32-pixel bands)
 #define DP_G(q) (KH == 1 ? (q) : 2 * (q) + hv)
@@ -2271,7 +2303,7 @@ __global__ __launch_bounds__(DP_NT, 1) void k_dparts(D8sPartsArgs a) {
     // prefetched state: conv1 tables of the next conv1 pass (t_abh, t_w1sum, t_gd), conv2 tables of the
     // next conv2 (t_w2, t_sc, t_w2sum), the weights of a layer's newest group (t_wn)
     u32x4 t_w2[5];
-    uint32_t t_abh[4];
+    u32x4 t_abh = {0u, 0u, 0u, 0u};
     int32_t t_w1sum = 0, t_w2sum = 0;
     float2 t_gd = {0.f, 0.f};
     float t_sc = 0.f;
@@ -2282,8 +2314,7 @@ __global__ __launch_bounds__(DP_NT, 1) void k_dparts(D8sPartsArgs a) {
         const int ti_ = min(tid, 127);                                                            \
         t_w1sum = ldg_i32((lp_).w1sum + ti_);                                                     \
         t_gd = ldg_f2((const float2*)(lp_).gd + ti_);                                             \
-        _Pragma("unroll") for (int k_ = 0; k_ < 4; ++k_)                                          \
-            t_abh[k_] = ldg_u32((const uint32_t*)(lp_).abh + min(tid + DP_NT * k_, (G_) * 32 - 1)); \
+        t_abh = ldg_u32x4((const u32x4*)(lp_).abh + min(tid, (G_) * 8 - 1));                      \
     } while (0)
 #define DP_TAB2(lp_)                                                                              \
     do {                                                                                          \
@@ -2295,22 +2326,34 @@ __global__ __launch_bounds__(DP_NT, 1) void k_dparts(D8sPartsArgs a) {
     } while (0)
     // weights of output tile c of group g (the MFMA A operand: rows 32 c + j, bytes 16 h ..)
 #define DP_W(lp_, g) ldg_u32x4((const uint8_t*)(lp_).w1 + ((int64_t)(g) * 128 + 32 * c + j) * 32 + 16 * h)
-#define DP_RW(lp_, G_)                                                                            \
-    _Pragma("unroll") for (int q_ = 0; q_ < DW; ++q_) rw[q_] = DP_W(lp_, min(DP_G(q_), (G_) - 1))
-    // store bytes of the items of chunk ch a wave prologues (item i = wave + 8 q: group i / PT, tile
-    // i % PT); `ready_` = groups that exist already
-#define DP_RA(ch_, G_, ready_)                                                                    \
-    _Pragma("unroll") for (int q_ = 0; q_ < IPW; ++q_) {                                          \
-        const int i_ = wave + 8 * q_, g_ = min((ch_) * CG + i_ / PT, (ready_) - 1);                \
-        ra[q_] = *(const u32x4*)DP_SRC(g_, i_ % PT);                                              \
-    }
+    // the same in the conv1 loop, as buffer loads of rw1_ (w1's G groups): a group past the last reads
+    // nothing and gives zeros
+    const uint32_t wl = (uint32_t)((32 * c + j) * 32 + 16 * h);
+#define DP_WB(g, G_) bload128(rw1_, wl + ((g) < (G_) ? (uint32_t)(g) * 4096u : DP_OOB), 0)
+#define DP_RW(G_)                                                                                 \
+    _Pragma("unroll") for (int q_ = 0; q_ < DW; ++q_) rw[q_] = DP_WB(DP_G(q_), G_)
+    // store bytes of the wave's items of chunk ch, as buffer loads: for a group past the `ready_` ones that
+    // exist already they read nothing (what no step uses costs no traffic)
+#define DP_RSRC(ch_, ready_)                                                                      \
+    brsrc(DP_GRP((ch_) * CG + pg), (ch_) * CG + pg < (ready_) ? (uint32_t)HW * 32u : 0u)
+#define DP_RA(ch_, ready_)                                                                        \
+    do {                                                                                          \
+        const __amdgpu_buffer_rsrc_t r_ = DP_RSRC(ch_, ready_);                                   \
+        _Pragma("unroll") for (int q_ = 0; q_ < IPW; ++q_) ra[q_] = bload128(r_, DP_OFF(q_), 0);  \
+    } while (0)
+    // a wave's 32 x 32 sums to and from partial-sum tile t_ (a dword per lane at a time: 16-byte rows were
+    // no faster for 32-pixel bands and 5 % slower for 64-pixel ones)
+#define DP_RED_PUT(t_, a_)                                                                        \
+    _Pragma("unroll") for (int v_ = 0; v_ < 16; ++v_) s_red[(t_) * 1024 + v_ * 64 + lane] = a_[v_]
+#define DP_RED_ADD(t_, a_)                                                                        \
+    _Pragma("unroll") for (int v_ = 0; v_ < 16; ++v_) a_[v_] += s_red[(t_) * 1024 + v_ * 64 + lane]
 #define DP_XCH_TAG(l_) ((uint64_t)(epoch * 64u + (uint32_t)(l_) + 1u) << 32)
 
     if (valid) {
         const D8sLayerP lp0 = DP_LP(0);
         DP_TAB1(lp0, G0);
         DP_TAB2(lp0);
-        DP_RA(0, G0, G0);
+        DP_RA(0, G0);
     }
     // Pass i: (A) conv1 of layer i over the groups that exist before layer i - 1's conv2 (all but the
     // newest), (B) layer i - 1's halo rows and its conv2, whose output (the newest group) goes
@@ -2318,6 +2361,18 @@ __global__ __launch_bounds__(DP_NT, 1) void k_dparts(D8sPartsArgs a) {
     // the window and its first / last rows out to the neighbours.  The neighbours' rows of layer i are
     // waited for only in pass i + 1, after its conv1: the exchange runs beside that conv1.
     i32x16 acc[NPT];
+    // the neighbours' rows of layer l into the halo rows (window row 0 = the band above's last row, row
+    // R + 1 = the band below's first row): a thread's first (value, tag) pairs, checked after the conv1 loop
+    uint64_t f[4] = {0, 0, 0, 0};
+#define DP_POLL(l_)                                                                               \
+    do {                                                                                          \
+        const int idx = min(tid, 16 * W - 1);                                                     \
+        const int hh = idx & 1, xx = (idx >> 1) % W, cc = ((idx >> 1) / W) & 3, below = idx / (8 * W); \
+        const bool has = below ? part < K - 1 : part > 0;                                         \
+        const int tk = has ? (below ? ticket + 1 : ticket - 1) : ticket;                          \
+        const uint64_t* xp = DP_XP(tk, (l_) & 1, below ? 0 : 1, cc) + xx * 8 + 4 * hh;            \
+        _Pragma("unroll") for (int e4 = 0; e4 < 4; ++e4) f[e4] = ld_agent64(xp + e4);             \
+    } while (0)
     for (int i = 0; i <= (valid ? L : -1); ++i) {
         // ==== (A) conv1 of layer i over its groups 0 .. G - 1 ====
         if (i < L) {
@@ -2338,29 +2393,24 @@ __global__ __launch_bounds__(DP_NT, 1) void k_dparts(D8sPartsArgs a) {
                 s_w1sum[tid] = t_w1sum;
                 s_gd[tid] = t_gd;
             }
-#pragma unroll
-            for (int k = 0; k < 4; ++k)
-                if (tid + DP_NT * k < (G0 + i) * 32) s_abh[tid + DP_NT * k] = t_abh[k];
+            if (tid < (G0 + i) * 8) ((u32x4*)s_abh)[tid] = t_abh;    // (at most 64 groups: 512 threads)
             // group G - 1 (layer i - 2's output), if it is in chunk 0, was not ready when chunk 0 was
             // requested: its bytes from the copy conv2 left in LDS (a global load here would make the
             // prologue below wait for every store in flight)
             if (i > 1 && G - 1 < CG) {
 #pragma unroll
-                for (int q_ = 0; q_ < IPW; ++q_) {
-                    const int i_ = wave + 8 * q_;
-                    if (i_ / PT == G - 1) ra[q_] = s_pro[(ITEMS + i_ % PT) * 64 + lane];
-                }
+                for (int q_ = 0; q_ < IPW; ++q_)
+                    if (pg == G - 1) ra[q_] = s_pro[(ITEMS + pt0 + q_) * 64 + lane];
             }
             __syncthreads();                               // tables in LDS
 
-            // ---- prologue of chunk ch into LDS buffer ch & 1 ----
-#define DP_PRO(ch_)                                                                               \
-    _Pragma("unroll") for (int q_ = 0; q_ < IPW; ++q_) {                                          \
-        const int i_ = wave + 8 * q_, g_ = min((ch_) * CG + i_ / PT, G - 1);                      \
-        const u32x4* pp_ = (const u32x4*)(s_abh + g_ * 32 + h * 16);                              \
-        s_pro[(((ch_) & 1) * ITEMS + i_) * 64 + lane] = pro16(ra[q_], pp_[0], pp_[1], pp_[2], pp_[3]); \
-    }
-            DP_PRO(0);
+            // ---- prologue of chunk 0 into LDS buffer 0 ----
+            {
+                const u32x4* pp_ = (const u32x4*)(s_abh + min(pg, G - 1) * 32 + h * 16);
+#pragma unroll
+                for (int q_ = 0; q_ < IPW; ++q_)
+                    s_pro[(pg * PT + pt0 + q_) * 64 + lane] = pro16(ra[q_], pp_[0], pp_[1], pp_[2], pp_[3]);
+            }
             // the next layer's conv1 tables and this layer's newest-group weights (unconditional, a
             // clamped layer: a load under a branch makes later waits wait for every load), then the
             // loads in the loop's order (activations two chunks ahead, then the weight ring), so the
@@ -2371,8 +2421,9 @@ __global__ __launch_bounds__(DP_NT, 1) void k_dparts(D8sPartsArgs a) {
                 DP_TAB1(ln, G0 + ln_);
                 t_wn = DP_W(lp, G0 + i - 1);                 // (i = 0: group G0 - 1, unused)
             }
-            DP_RA(1, G, G);
-            DP_RW(lp, G);
+            DP_RA(1, G);
+            const __amdgpu_buffer_rsrc_t rw1_ = brsrc((const void*)uniform64((uint64_t)lp.w1), (uint32_t)G * 4096u);
+            DP_RW(G);
             __syncthreads();
             const int32_t m128 = hv == 0 || KH == 1 ? 128 : 0;      // one K half starts at 128 sum w
 #pragma unroll
@@ -2380,53 +2431,61 @@ __global__ __launch_bounds__(DP_NT, 1) void k_dparts(D8sPartsArgs a) {
 #pragma unroll
                 for (int v = 0; v < 16; ++v) acc[tt][v] = m128 * s_w1sum[32 * c + res_row(v, h)];
             }
-            for (int ch = 0; ch < nch; ++ch) {
-                // straight-line steps (no load under a branch: the wait counts stay exact and the
-                // prefetched loads stay in flight); a step past the last group multiplies zero weights.
-                // The next chunk's prologue items are spread between the steps, so their VALU work runs
-                // beside the MFMAs already issued (an item past the last chunk is never read).
-                const u32x4* bsrc = s_pro + (ch & 1) * ITEMS * 64 + lane;
-                constexpr int EVERY = QC / IPW;            // steps per prologue item
-                // the chunk's operands read from LDS together, so the steps wait for one latency (where
-                // the registers allow: up to 8 operands)
-                constexpr bool BX = QC * NPT <= 8;
-                u32x4 bx[BX ? QC : 1][BX ? NPT : 1];
-                if constexpr (BX) {
-#pragma unroll
-                    for (int u = 0; u < QC; ++u) {
-                        const int gi = (KH == 2 ? 2 * u + hv : u);
-#pragma unroll
-                        for (int tt = 0; tt < NPT; ++tt)
-                            bx[u][tt] = bsrc[(gi * PT + (KH == 2 ? 0 : hv * NPT + tt)) * 64];
-                    }
-                }
-#pragma unroll
-                for (int u = 0; u < QC; ++u) {
-                    const int q = ch * QC + u, g = DP_G(q);
-                    const uint32_t live = g < G ? ~0u : 0u;
-                    const u32x4 wa = rw[u % DW] & u32x4{live, live, live, live};
-                    rw[u % DW] = DP_W(lp, min(DP_G(q + DW), G - 1));
-                    const int gi = (KH == 2 ? 2 * u + hv : u);
-#pragma unroll
-                    for (int tt = 0; tt < NPT; ++tt) {
-                        const int t = KH == 2 ? 0 : hv * NPT + tt;
-                        acc[tt] = mfma_i8(wa, BX ? bx[BX ? u : 0][BX ? tt : 0] : bsrc[(gi * PT + t) * 64], acc[tt]);
-                    }
-                    if ((u + 1) % EVERY == 0) {
-                        const int qi = (u + 1) / EVERY - 1;    // item wave + 8 qi of chunk ch + 1
-                        const int i_ = wave + 8 * qi, g_ = min((ch + 1) * CG + i_ / PT, G - 1);
-                        const u32x4* pp_ = (const u32x4*)(s_abh + g_ * 32 + h * 16);
-                        s_pro[(((ch + 1) & 1) * ITEMS + i_) * 64 + lane] =
-                            pro16(ra[qi], pp_[0], pp_[1], pp_[2], pp_[3]);
-                        const int g2 = min((ch + 2) * CG + i_ / PT, G - 1);
-                        ra[qi] = *(const u32x4*)DP_SRC(g2, i_ % PT);
-                    }
-                    __builtin_amdgcn_sched_barrier(0);
-                }
-                __syncthreads();                           // chunk ch read, chunk ch + 1 written
-            }
+            // straight-line steps (no load under a branch: the wait counts stay exact and the prefetched
+            // loads stay in flight); a step past the last group multiplies zero weights.  The next chunk's
+            // prologue items are spread between the steps, so their VALU work runs beside the MFMAs
+            // already issued.  The chunk's operands are read from LDS together, so the steps wait for one
+            // latency (where the registers allow: up to 8 operands).  pre_ = whether a chunk follows (its
+            // prologue and the loads ahead: the last chunk issues none)
+            constexpr bool BX = QC * NPT <= 8;
+            constexpr int EVERY = QC / IPW;                // steps per prologue item
+            constexpr bool TP = IPW == 2 || IPW == 3;      // the items' table read once per chunk
+#define DP_CHUNK(ch_, pre_)                                                                       \
+    do {                                                                                          \
+        const u32x4* bsrc = s_pro + ((ch_) & 1) * ITEMS * 64 + lane;                              \
+        u32x4 bx[BX ? QC : 1][BX ? NPT : 1];                                                      \
+        if constexpr (BX) {                                                                       \
+            _Pragma("unroll") for (int u = 0; u < QC; ++u) {                                      \
+                const int gi = (KH == 2 ? 2 * u + hv : u);                                        \
+                _Pragma("unroll") for (int tt = 0; tt < NPT; ++tt)                                \
+                    bx[u][tt] = bsrc[(gi * PT + (KH == 2 ? 0 : hv * NPT + tt)) * 64];             \
+            }                                                                                     \
+        }                                                                                         \
+        const u32x4* pp_ = (const u32x4*)(s_abh + min(((ch_) + 1) * CG + pg, G - 1) * 32 + h * 16); \
+        u32x4 pt_[TP ? 4 : 1];                                                                    \
+        if constexpr (TP && (pre_)) {                                                             \
+            _Pragma("unroll") for (int k_ = 0; k_ < 4; ++k_) pt_[k_] = pp_[k_];                   \
+        }                                                                                         \
+        const __amdgpu_buffer_rsrc_t gr_ = DP_RSRC((ch_) + 2, G);                                 \
+        _Pragma("unroll") for (int u = 0; u < QC; ++u) {                                          \
+            const int q = (ch_) * QC + u;                                                         \
+            const u32x4 wa = rw[u];                                                          \
+            if (pre_) rw[u] = DP_WB(DP_G(q + DW), G);                                        \
+            const int gi = (KH == 2 ? 2 * u + hv : u);                                            \
+            _Pragma("unroll") for (int tt = 0; tt < NPT; ++tt) {                                  \
+                const int t = KH == 2 ? 0 : hv * NPT + tt;                                        \
+                acc[tt] = mfma_i8(wa, BX ? bx[BX ? u : 0][BX ? tt : 0] : bsrc[(gi * PT + t) * 64], acc[tt]); \
+            }                                                                                     \
+            if ((pre_) && (u + 1) % EVERY == 0 && (u + 1) / EVERY <= IPW) {                       \
+                const int qi = (u + 1) / EVERY - 1;                                               \
+                s_pro[((((ch_) + 1) & 1) * ITEMS + pg * PT + pt0 + qi) * 64 + lane] =             \
+                    TP ? pro16(ra[qi], pt_[0], pt_[TP ? 1 : 0], pt_[TP ? 2 : 0], pt_[TP ? 3 : 0]) \
+                       : pro16(ra[qi], pp_[0], pp_[1], pp_[2], pp_[3]);                      \
+                ra[qi] = bload128(gr_, DP_OFF(qi), 0);                                           \
+            }                                                                                     \
+            __builtin_amdgcn_sched_barrier(0);                                                    \
+        }                                                                                         \
+        __syncthreads();                                   /* chunk read, the next one written */ \
+    } while (0)
+            // the neighbours' rows are requested before the last chunk, whose loads are all older (loads
+            // complete in order): their round trip through the coherence point, about 1.3 us, runs beside
+            // that chunk.  Requested after the loop it took 13-19 % of the layer
+            for (int ch = 0; ch + 1 < nch; ++ch) DP_CHUNK(ch, true);
+            if (!RAG || K > 1) DP_POLL(i - 1);
+            DP_CHUNK(nch - 1, false);
+#undef DP_CHUNK
             // the next pass's first chunk: its groups but the newest exist (that one: see above)
-            DP_RA(0, G0 + i, G);
+            DP_RA(0, G);
         }
 
         // ==== (B) layer i - 1's halo rows and conv2 ====
@@ -2438,11 +2497,11 @@ __global__ __launch_bounds__(DP_NT, 1) void k_dparts(D8sPartsArgs a) {
             // conv2's pixel tile t2 and K steps st = s2, s2 + S2, ... of 36 for this wave; a tile whose
             // rows all lie inside the band (rows 1 .. R - 2) reads no halo row, so its MFMAs run while
             // the neighbours' rows are read
-            const bool active = PT == 1 ? wave < 4 : true;
             const int t2 = PT == 1 ? 0 : wave / S2, s2 = PT == 1 ? wave : wave % S2;
-            const int pl = 32 * t2 + j, yl = pl / W, x = pl - yl * W;
+            const bool active = (PT == 1 ? wave < 4 : PT == 6 ? wave < 6 : true) && (!RAG || 32 * t2 < P);
+            const int pl = 32 * t2 + j, pc = RAG ? min(pl, P - 1) : pl, yl = pc / W, x = pc - yl * W;
             const int q0 = yl * BW + x;
-            const bool inner = (32 * t2) / W >= 1 && (32 * t2 + 31) / W <= R - 2;
+            const bool inner = (32 * t2) / W >= 1 && (RAG ? min(32 * t2 + 31, P - 1) : 32 * t2 + 31) / W <= R - 2;
             i32x16 acc2;
 #pragma unroll
             for (int v = 0; v < 16; ++v) acc2[v] = s2 == 0 ? 128 * s_w2sum[res_row(v, h)] : 0;
@@ -2467,19 +2526,9 @@ __global__ __launch_bounds__(DP_NT, 1) void k_dparts(D8sPartsArgs a) {
             __builtin_amdgcn_sched_barrier(0);                                                    \
         }                                                                                         \
     } while (0)
-            // the neighbours' rows into the halo rows (window row 0 = the band above's last row, row
-            // R + 1 = the band below's first row), polling each pair until its tag is current; a
-            // thread's first pair is read before the inner tiles' MFMAs (an edge band reads its own
-            // pairs there, unused)
-            uint64_t f[4];
-            {
-                const int idx = min(tid, 16 * W - 1);
-                const int hh = idx & 1, xx = (idx >> 1) % W, cc = ((idx >> 1) / W) & 3, below = idx / (8 * W);
-                const bool has = below ? part < K - 1 : part > 0;
-                const int tk = has ? (below ? ticket + 1 : ticket - 1) : ticket;
-                const uint64_t* xp = DP_XP(tk, par, below ? 0 : 1, cc) + xx * 8 + 4 * hh;
-#pragma unroll
-                for (int e4 = 0; e4 < 4; ++e4) f[e4] = ld_agent64(xp + e4);
+            // (the last pass has no conv1 loop to read its first pairs before)
+            if (i == L && (!RAG || K > 1)) {
+                DP_POLL(lc);
             }
             if (active && inner) {
                 DP_CONV2();
@@ -2522,18 +2571,12 @@ __global__ __launch_bounds__(DP_NT, 1) void k_dparts(D8sPartsArgs a) {
             }
             if constexpr (S2 > 1) {
                 if (active && s2 > 0) {
-                    int32_t* r = s_red + ((s2 - 1) * PT + t2) * 1024 + lane;
-#pragma unroll
-                    for (int v = 0; v < 16; ++v) r[v * 64] = acc2[v];
+                    DP_RED_PUT((s2 - 1) * PT + t2, acc2);
                 }
                 __syncthreads();
                 if (active && s2 == 0) {
 #pragma unroll
-                    for (int qq = 1; qq < S2; ++qq) {
-                        const int32_t* r = s_red + ((qq - 1) * PT + t2) * 1024 + lane;
-#pragma unroll
-                        for (int v = 0; v < 16; ++v) acc2[v] += r[v * 64];
-                    }
+                    for (int qq = 1; qq < S2; ++qq) DP_RED_ADD((qq - 1) * PT + t2, acc2);
                 }
             }
             if (active && s2 == 0) {
@@ -2541,7 +2584,7 @@ __global__ __launch_bounds__(DP_NT, 1) void k_dparts(D8sPartsArgs a) {
 #pragma unroll
                 for (int kk = 0; kk < 4; ++kk) e[kk] = epi2_q(acc2, kk, *(const float4*)(s_sc + 8 * kk + 4 * h));
                 const u32x4 row = xchg_rows(e[0], e[1], e[2], e[3], h);
-                *(u32x4*)(segn + (int64_t)lc * slot + (uint32_t)((bandp + pl) * 32 + 16 * h)) = row;
+                if (!RAG || pl < P) *(u32x4*)(segn + (int64_t)lc * slot + (uint32_t)((bandp + pl) * 32 + 16 * h)) = row;
                 // the new group's bytes of pixel tile t2 through layer i's prologue: exactly the MFMA B
                 // operand of that tile (pixel j, bytes 16 h ..)
                 if (i < L) {
@@ -2577,17 +2620,9 @@ __global__ __launch_bounds__(DP_NT, 1) void k_dparts(D8sPartsArgs a) {
             }
             // 32-pixel bands: the two K halves of each output tile added through LDS
             if constexpr (KH == 2) {
-                if (hv == 1) {
-                    int32_t* r = s_red + c * 1024 + lane;
-#pragma unroll
-                    for (int v = 0; v < 16; ++v) r[v * 64] = acc[0][v];
-                }
+                if (hv == 1) DP_RED_PUT(c, acc[0]);
                 __syncthreads();
-                if (hv == 0) {
-                    const int32_t* r = s_red + c * 1024 + lane;
-#pragma unroll
-                    for (int v = 0; v < 16; ++v) acc[0][v] += r[v * 64];
-                }
+                if (hv == 0) DP_RED_ADD(c, acc[0]);
             }
             // ---- bottleneck bytes (v ^ 0x80) into the window; the band's first / last row out ----
             const int par = i & 1;
@@ -2604,8 +2639,8 @@ __global__ __launch_bounds__(DP_NT, 1) void k_dparts(D8sPartsArgs a) {
                         e[kk] = epi1_x80(acc[tt], kk, pg[0], pg[1]);
                     }
                     const u32x4 row = xchg_rows(e[0], e[1], e[2], e[3], h);
-                    s_b[c * WIN * 2 + swz((yl + 1) * BW + x + 1, h)] = row;
-                    if (yl == 0 && part > 0) {
+                    if (!RAG || pl < P) s_b[c * WIN * 2 + swz((yl + 1) * BW + x + 1, h)] = row;
+                    if (yl == 0 && part > 0) {                 // (a lane past the band has yl >= R >= 1)
                         uint64_t* xp = DP_XP(ticket, par, 0, c) + x * 8 + 4 * h;
 #pragma unroll
                         for (int e4 = 0; e4 < 4; ++e4) st_agent64(xp + e4, tag | row[e4]);
@@ -2620,17 +2655,23 @@ __global__ __launch_bounds__(DP_NT, 1) void k_dparts(D8sPartsArgs a) {
             }
         }
     }
-#undef DP_PRO
 #undef DP_RA
 #undef DP_RW
 #undef DP_W
+#undef DP_WB
 #undef DP_TAB1
 #undef DP_TAB2
 #undef DP_XCH_TAG
+#undef DP_POLL
 #undef DP_LP
 #undef DP_G
 #undef DP_XP
-#undef DP_SRC
+#undef DP_LDA
+#undef DP_GRP
+#undef DP_OFF
+#undef DP_RSRC
+#undef DP_RED_PUT
+#undef DP_RED_ADD
     // the last workgroup to end resets the ticket and the end count, and counts the launch
     if (tid == 0) {
         const uint32_t done = __hip_atomic_fetch_add(sync + 1, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
@@ -3976,25 +4017,79 @@ extern "C" int d8s_dense_block_pair(const D8sBlockArgs* a, const D8sBlockArgs* b
     return dblock_launch(a, b, (hipStream_t)stream);
 }
 
+// LDS of a banded whole block: the window of R + 2 rows of W + 2 pixels (4 planes), the layer tables and
+// the prologue tables (dynamic), and k_dparts<PT>'s static arrays.
+static size_t parts_static(int PT) {
+    return PT == 1 ? DpShape<1>::STATIC : PT == 2 ? DpShape<2>::STATIC : PT == 4 ? DpShape<4>::STATIC
+         : PT == 6 ? DpShape<6>::STATIC : DpShape<8>::STATIC;
+}
+static size_t parts_dyn(int R, int W, int G) { return (size_t)(R + 2) * (W + 2) * 128 + DB_PRM + (size_t)G * 128; }
+
 // The shape checks of d8s_dense_block_parts (H, W, groups read by the last layer, bands per image):
-// nullptr if it runs, else the reason; *shm = its dynamic LDS bytes.
-static const char* parts_shape(int H, int W, int G, int parts, size_t* shm) {
+// nullptr if it runs, else the reason; *shm = its dynamic LDS bytes, *PT = its pixel tiles per band.
+static const char* parts_shape(int H, int W, int G, int parts, size_t* shm, int* PT) {
     if (H < 1 || W < 1 || G < 1 || parts < 1) return "H, W, groups and parts must be >= 1";
     if (H % parts) return "H must be a multiple of parts";
-    const int R = H / parts, P = R * W;
+    const int R = H / parts;
+    const int64_t P = (int64_t)R * W;
     if (P != 32 && P != 64 && P != 128 && P != 256) return "(H / parts) * W must be 32, 64, 128 or 256 pixels";
     if (G > 64) return "more than 64 groups";
-    // the band's window (R + 2 rows of W + 2 pixels, 4 planes), the layer tables, the prologue tables
-    const size_t dyn = (size_t)(R + 2) * (W + 2) * 128 + DB_PRM + (size_t)G * 128;
-    const size_t stat = P == 32 ? DpShape<1>::STATIC : P == 64 ? DpShape<2>::STATIC
-                      : P == 128 ? DpShape<4>::STATIC : DpShape<8>::STATIC;
-    if (dyn + stat > 160 * 1024) return "band too large for LDS";
+    const size_t dyn = parts_dyn(R, W, G);
+    if (dyn + parts_static((int)(P / 32)) > 160 * 1024) return "band too large for LDS";
     if (shm) *shm = dyn;
+    if (PT) *PT = (int)(P / 32);
+    return nullptr;
+}
+
+// The same of d8s_dense_block_bands: any split into at most H bands of at most 256 pixels.
+static const char* bands_shape(int H, int W, int G, int bands, size_t* shm, int* PT) {
+    if (H < 1 || W < 1 || G < 1 || bands < 1) return "H, W, groups and bands must be >= 1";
+    if (bands > H) return "more bands than rows";
+    const int R = (H - 1) / bands + 1;
+    if ((int64_t)R * W > 256) return "a band has more than 256 pixels";
+    if (G > 64) return "more than 64 groups";
+    const int t = (R * W + 31) / 32, pt = t <= 2 ? t : (t + 1) / 2 * 2;     // 1, 2, 4, 6 or 8 pixel tiles
+    const size_t dyn = parts_dyn(R, W, G);
+    if (dyn + parts_static(pt) > 160 * 1024) return "band too large for LDS";
+    if (shm) *shm = dyn;
+    if (PT) *PT = pt;
     return nullptr;
 }
 
 extern "C" int d8s_parts_supported(int32_t H, int32_t W, int32_t G, int32_t parts) {
-    return parts_shape(H, W, G, parts, nullptr) == nullptr ? 1 : 0;
+    return parts_shape(H, W, G, parts, nullptr, nullptr) == nullptr ? 1 : 0;
+}
+
+extern "C" int d8s_bands_supported(int32_t H, int32_t W, int32_t G, int32_t bands) {
+    return bands_shape(H, W, G, bands, nullptr, nullptr) == nullptr ? 1 : 0;
+}
+
+// Checks the arguments both banded entry points share, then launches k_dparts<PT, rag>.
+static int parts_launch(const D8sPartsArgs* a, int PT, bool rag, size_t shm, hipStream_t st, const char* what) {
+    const std::string w(what);
+    REQUIRE((int64_t)a->N * a->parts < (1 << 24), w + ": too many parts");
+    REQUIRE((int64_t)a->N * a->H * a->W * 32 < (1ll << 31), w + ": store slot over 2 GiB");
+    REQUIRE(a->parts <= cu_count(), w + ": more bands per image than compute units");
+    typedef void (*Kernel)(D8sPartsArgs);
+    static const Kernel KERNELS[2][5] = {
+        {k_dparts<1, false>, k_dparts<2, false>, k_dparts<4, false>, nullptr, k_dparts<8, false>},
+        {k_dparts<1, true>, k_dparts<2, true>, k_dparts<4, true>, k_dparts<6, true>, k_dparts<8, true>}};
+    const Kernel fn = KERNELS[rag][PT / 2];
+    REQUIRE(fn != nullptr, w + ": no kernel of this band size");
+    // the LDS check counts parts_static bytes of static LDS: make sure the compiled kernel uses no more
+    // (checked once per kernel; the check has no side effect, so threads may repeat it)
+    {
+        static std::atomic<bool> checked[2][5];
+        if (!checked[rag][PT / 2]) {
+            hipFuncAttributes at{};
+            const hipError_t e = hipFuncGetAttributes(&at, (const void*)fn);
+            if (e != hipSuccess) return fail((int)e, w + ": " + hipGetErrorString(e));
+            REQUIRE(at.sharedSizeBytes <= parts_static(PT), w + ": the kernel's static LDS exceeds its estimate");
+            checked[rag][PT / 2] = true;
+        }
+    }
+    hipLaunchKernelGGL(fn, dim3((unsigned)(a->N * a->parts)), dim3(DP_NT), shm, st, *a);
+    return launched(what);
 }
 
 extern "C" int d8s_dense_block_parts(const D8sPartsArgs* a, void* stream) {
@@ -4003,38 +4098,21 @@ extern "C" int d8s_dense_block_parts(const D8sPartsArgs* a, void* stream) {
     REQUIRE(a->G0 >= 1 && a->L >= 1 && a->N >= 1 && a->H >= 1 && a->W >= 1 && a->parts >= 1,
             "d8s_dense_block_parts: G0, L, N, H, W, parts must be >= 1");
     size_t shm = 0;
-    const char* why = parts_shape(a->H, a->W, a->G0 + a->L - 1, a->parts, &shm);
+    int PT = 0;
+    const char* why = parts_shape(a->H, a->W, a->G0 + a->L - 1, a->parts, &shm, &PT);
     REQUIRE(why == nullptr, std::string("d8s_dense_block_parts: ") + (why ? why : ""));
-    REQUIRE((int64_t)a->N * a->parts < (1 << 24), "d8s_dense_block_parts: too many parts");
-    REQUIRE((int64_t)a->N * a->H * a->W * 32 < (1ll << 31), "d8s_dense_block_parts: store slot over 2 GiB");
-    REQUIRE(a->parts <= cu_count(), "d8s_dense_block_parts: more bands per image than compute units");
-    const int P = (a->H / a->parts) * a->W;
-    // the LDS check above counts DpShape<PT>::STATIC bytes of static LDS: make sure the compiled kernel
-    // uses no more (checked once per band size)
-    {
-        static int checked[9] = {0};
-        const int PT = P / 32;
-        if (!checked[PT]) {
-            hipFuncAttributes at{};
-            const void* fn = PT == 1 ? (const void*)k_dparts<1> : PT == 2 ? (const void*)k_dparts<2>
-                           : PT == 4 ? (const void*)k_dparts<4> : (const void*)k_dparts<8>;
-            const size_t want = PT == 1 ? DpShape<1>::STATIC : PT == 2 ? DpShape<2>::STATIC
-                              : PT == 4 ? DpShape<4>::STATIC : DpShape<8>::STATIC;
-            const hipError_t e = hipFuncGetAttributes(&at, fn);
-            if (e != hipSuccess) return fail((int)e, std::string("d8s_dense_block_parts: ") + hipGetErrorString(e));
-            REQUIRE(at.sharedSizeBytes <= want, "d8s_dense_block_parts: the kernel's static LDS exceeds its estimate");
-            checked[PT] = 1;
-        }
-    }
-    hipStream_t st = (hipStream_t)stream;
-    const dim3 grid((unsigned)(a->N * a->parts));
-    switch (P / 32) {
-        case 1: hipLaunchKernelGGL(k_dparts<1>, grid, dim3(DP_NT), shm, st, *a); break;
-        case 2: hipLaunchKernelGGL(k_dparts<2>, grid, dim3(DP_NT), shm, st, *a); break;
-        case 4: hipLaunchKernelGGL(k_dparts<4>, grid, dim3(DP_NT), shm, st, *a); break;
-        default: hipLaunchKernelGGL(k_dparts<8>, grid, dim3(DP_NT), shm, st, *a); break;
-    }
-    return launched("d8s_dense_block_parts");
+    return parts_launch(a, PT, false, shm, (hipStream_t)stream, "d8s_dense_block_parts");
+}
+
+extern "C" int d8s_dense_block_bands(const D8sPartsArgs* a, void* stream) {
+    REQUIRE(a != nullptr, "d8s_dense_block_bands: null arguments");
+    REQUIRE(a->in0 && a->seg && a->layers && a->sync && a->xchg, "d8s_dense_block_bands: null pointer");
+    REQUIRE(a->G0 >= 1 && a->L >= 1 && a->N >= 1, "d8s_dense_block_bands: G0, L, N must be >= 1");
+    size_t shm = 0;
+    int PT = 0;
+    const char* why = bands_shape(a->H, a->W, a->G0 + a->L - 1, a->parts, &shm, &PT);
+    REQUIRE(why == nullptr, std::string("d8s_dense_block_bands: ") + (why ? why : ""));
+    return parts_launch(a, PT, true, shm, (hipStream_t)stream, "d8s_dense_block_bands");
 }
 
 template <int NT, int PT, int D, int WB>

@@ -595,8 +595,10 @@ def contents_id(x: torch.Tensor) -> tuple:
 # layer (d8s_dense, the reference's fused kind "tile"); "img" the whole block in one launch, a workgroup
 # per image (d8s_dense_block, the reference's "img*" kinds); "parts" the whole block in one launch with
 # every image split into row bands, a workgroup per band (d8s_dense_block_parts; "parts:K" for K bands,
-# plain "parts" for as many as fill the chip).  The bytes are the same.
-BLOCK_KINDS = ("conv", "chain", "tile", "img", "parts")
+# plain "parts" for as many as fill the chip); "bands:K" the same with bands of any row count and width
+# (d8s_dense_block_bands, for maps whose rows make no whole 32-pixel tiles).  The bytes are the same.
+BLOCK_KINDS = ("conv", "chain", "tile", "img", "parts", "bands")
+BANDED_ENTRIES = ("d8s_dense_block_parts", "d8s_dense_block_bands")
 IMG_MAX_PX = 256                # d8s_dense_block: pixels per image
 IMG_MAX_GROUPS = 64             # and groups read by the last layer
 # the reference's fused kinds (`src/knee/dense8s.py:174-176`) as this runner's: its whole-block kinds
@@ -627,6 +629,15 @@ def parts_for(b: dict, n: int, cus: int = 256) -> int | None:
     workgroups (one workgroup per CU: its LDS), or None if no split fits."""
     fit = [k for k in parts_options(b) if n * k <= cus]
     return fit[-1] if fit else None
+
+
+def bands_options(b: dict) -> list[int]:
+    """Band counts d8s_dense_block_bands can split block `b`'s images into (increasing), the least for each
+    number of rows, without the ones `parts_options` has."""
+    lib = hip.library()
+    h, g = b["h"], block_groups(b)
+    counts = sorted({-(-h // rows) for rows in range(1, h + 1)} - set(parts_options(b)))
+    return [k for k in counts if lib.d8s_bands_supported(h, b["w"], g, k)]
 
 
 def _kind_name(kind) -> str:
@@ -684,28 +695,62 @@ def recorded_variants(meta: dict) -> dict:
     return out
 
 
+def kind_us(b: dict, kind: str, n: int, cus: int = 256) -> float:
+    """Estimated us per layer of block `b` (meta) run as `kind` at n images per pass: what `tune_kinds`
+    measured on an MI355X over 1-96 images of 96-512 px, as lines in the mean group count g of the
+    block's layers, its pixels (kpx, thousands) and its rounds of workgroups (one per CU at a time).
+      bands / parts  a round costs the band's pixel tiles (6.4, 8.1, 10, 13 and 15 us a layer for 1, 2, 4,
+                     6 and 8 tiles at g = 23), whatever the count of bands that fit it, and the rows its
+                     workgroups exchange (0.3 us per thousand pixels of them);
+      img            14.4 us a round at g = 35;
+      chain          a launch of 8.6 us at g = 9 and 13 us per full round of three workgroups per CU;
+      tile           rounds of 32 x 12 (narrower maps: 16 x 12) tiles, 3.8 + 13 us (3.8 + 7.7) at g = 9;
+                     64 and 128 wide: rounds of row bands (`_band_steps`);
+      conv           two launches, 12 us at g = 9 (16 beyond one round), and their bytes, conv2's with its
+                     32 x 8 tiles' padding."""
+    h, w, g = b["h"], b["w"], b["c0"] / GROUP + (b["L"] - 1) / 2
+    kpx = n * h * w / 1000
+    name = _kind_name(kind)
+    if name in ("bands", "parts"):
+        k = int(kind.split(":", 1)[1])
+        tiles = -(-(-(-h // k) * w) // 32)
+        base, per_g = next(v for t, v in BAND_US if tiles <= t)
+        exchange = 0.3 * min(n * k, cus) * w / 1000 if k > 1 else 0.0
+        return -(-n * k // cus) * (base + per_g * g + exchange)
+    if name == "img":
+        return -(-n // cus) * (5.2 + 0.26 * g)
+    if name == "chain":
+        return 6.2 + 0.25 * g + 13.2 * kpx / (0.384 * cus)
+    if name == "tile":
+        if w in (64, 128) and block_groups(b) <= BAND_MAX_GROUPS:
+            return 1.5 + 0.55 * g + (0.95 + 0.1 * g) * w / 64 * _band_steps(h, w, n, cus)
+        tx, ty = (32, 12) if w >= 32 else (16, 16 if w <= 16 and h <= 16 else 12)
+        rounds = -(-n * -(-w // tx) * -(-h // ty) // cus)
+        return 3.8 + rounds * (8.0 + 0.53 * g if tx == 32 else 4.5 + 0.34 * g)
+    pad = -(-w // 32) * 32 / w * -(-h // 8) * 8 / h - 1
+    return 9.9 + 0.2 * g + (4.0 if kpx > 20 else 0.0) + (0.09 + 0.002 * g + 0.06 * pad) * kpx
+
+
+def _band_steps(h: int, w: int, n: int, cus: int) -> int:
+    """The rows d8s_dense's row bands walk in turn, all rounds together: the least of rounds x (rows + 2)
+    over the band heights the library chooses from."""
+    step = 256 // w
+    return min(-(-n * -(-h // r) // cus) * (r + 2) for r in range(step, 33, step))
+
+
+# (pixel tiles up to, (us per layer, us per group)) of a round of banded workgroups
+BAND_US = ((1, (5.9, 0.02)), (2, (7.0, 0.045)), (4, (8.6, 0.07)), (6, (10.0, 0.11)), (8, (11.6, 0.16)))
+
+
 def default_kind(b: dict, n: int, cus: int = 256) -> str:
-    """The block kind of block `b` at n images per pass: "parts" (the whole block in one launch, images
-    split into as many bands as fill the chip) where that takes 4 bands or more and the block either
-    fits a workgroup per image (the 16 x 16 maps of a 24-image study: 0.31 ms against 0.49 ms on 24
-    CUs) or splits into 8 bands (the 32 x 32 block of a 24-image study: one launch instead of 64
-    latency-bound ones); "img" where a workgroup per image fits (at 96 images: its 96 workgroups leave
-    room for a second encoder's pass on another stream, which 2-band launches of 192 did not); "tile"
-    for 128-wide blocks (the fused layer's band form); "chain" where the block's 128-pixel tiles fill
-    one round of three workgroups per CU to at least two thirds (the 32 x 32 block at 96 images: 0.82
-    against 0.89 ms per pass; the 64 x 64 block at 24 images: 0.24 against 0.26 ms; at 96 images that
-    block's four tiles per workgroup run slower chained than as two launches); else "conv"."""
-    k = parts_for(b, n, cus)
-    if k is not None and k >= 4 and (img_fits(b) or k >= 8):
-        return f"parts:{k}"
-    if img_fits(b):
+    """The block kind of block `b` at n images per pass: the least `kind_us` of the kinds it can take
+    (ties to the earlier one).  A map of a whole workgroup's 256 pixels whose images make more than a
+    quarter of the CUs stays "img" though two bands per image are faster alone: its one workgroup per
+    image leaves room for a second encoder's pass on another stream, which 2-band launches did not
+    (5.8 against 6.3-6.8 ms per study of two seeds at 96 images)."""
+    if img_fits(b) and b["h"] * b["w"] == IMG_MAX_PX and cus < 4 * n <= 4 * cus:
         return "img"
-    if band_fits(b):
-        return "tile"
-    tiles = n * b["h"] * b["w"] // 128
-    if chain_fits(b) and 2 * cus < tiles <= 3 * cus:
-        return "chain"
-    return "conv"
+    return min(kind_options(b, n), key=lambda kind: kind_us(b, kind, n, cus))
 
 
 def valid_kind(b: dict, bi: int, kind, n: int, cus: int = 256) -> str:
@@ -725,6 +770,12 @@ def valid_kind(b: dict, bi: int, kind, n: int, cus: int = 256) -> str:
             raise ValueError(f"block {bi} ({b['h']} x {b['w']}, {b['L']} layers) does not split into "
                              f"{k} bands (options {parts_options(b)})")
         return f"parts:{k}"
+    if name == "bands":
+        k = int(str(kind).split(":", 1)[1]) if ":" in str(kind) else 0
+        if not hip.library().d8s_bands_supported(b["h"], b["w"], block_groups(b), k):
+            raise ValueError(f"block {bi} ({b['h']} x {b['w']}, {b['L']} layers) does not split into "
+                             f"{k} bands (options {bands_options(b)})")
+        return f"bands:{k}"
     return name
 
 
@@ -773,6 +824,7 @@ def kind_options(b: dict, n: int) -> list[str]:
     if img_fits(b):
         out.append("img")
     out += [f"parts:{k}" for k in parts_options(b)]
+    out += [f"bands:{k}" for k in bands_options(b)]
     return out
 
 
@@ -1204,7 +1256,7 @@ class Dense8SEncoder(_PassRunner):
         """The launches of block bi's layers run as `kind`."""
         b = self.meta["blocks"][bi]
         L, name = b["L"], _kind_name(kind)
-        if name in ("img", "parts"):
+        if name in ("img", "parts", "bands"):
             g0 = b["c0"] // GROUP
             makes = tuple((bi, j) for j in range(1, L + 1))
             if name == "img":
@@ -1217,7 +1269,7 @@ class Dense8SEncoder(_PassRunner):
                                                                       device=f"cuda:{self.dev}"))
             args = hip.PartsArgs(self.in0[bi], self.seg[bi], self._layer_table(bi), _ptr(self._sync),
                                  _ptr(xchg), self.nb, b["h"], b["w"], g0, L, k)
-            return [Step("block", bi, -1, makes, "d8s_dense_block_parts", args)]
+            return [Step("block", bi, -1, makes, f"d8s_dense_block_{name}", args)]
         if name == "tile":
             steps = []
             for li in range(L):
@@ -1270,9 +1322,9 @@ class Dense8SEncoder(_PassRunner):
                                      f"taken for this shape")
                 step.variant = v
         self.program = prog
-        self._checked = any(s.entry == "d8s_dense_block_parts" for s in prog)
+        self._checked = any(s.entry in BANDED_ENTRIES for s in prog)
         # bands per image of the widest banded launch: its share of the CUs a wait needs resident
-        self.max_bands = max((s.args.parts for s in prog if s.entry == "d8s_dense_block_parts"), default=0)
+        self.max_bands = max((s.args.parts for s in prog if s.entry in BANDED_ENTRIES), default=0)
         if self._checked and self._report is None:
             # a host-mapped word the final kernel copies the banded blocks' error count into
             self._report = torch.zeros(2, dtype=torch.int32).pin_memory()

@@ -166,6 +166,8 @@ SIGNATURES = {
     "d8s_c21_supported": [i32, i32, i32],
     "d8s_dense_block": [ctypes.POINTER(BlockArgs), vp],
     "d8s_dense_block_parts": [ctypes.POINTER(PartsArgs), vp],
+    "d8s_dense_block_bands": [ctypes.POINTER(PartsArgs), vp],
+    "d8s_bands_supported": [i32, i32, i32, i32],
     "d8s_transition": [ctypes.POINTER(GemmArgs), vp],
     "d8s_final": [vp, i32, vp, i32, i32, vp, vp, i32, vp],
     "d8s_final_checked": [vp, i32, vp, i32, i32, vp, vp, i32, vp, vp, vp],

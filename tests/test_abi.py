@@ -66,6 +66,26 @@ def test_parts_supported_matches_the_launch():
     assert "LDS" in lib.d8s_last_error().decode()
 
 
+def test_bands_supported_matches_the_launch():
+    """d8s_bands_supported: any split into at most H bands of at most 256 pixels within LDS and 64
+    groups; what it refuses fails on the host."""
+    lib = hip.library()
+    assert lib.d8s_bands_supported(9, 9, 51, 1) == 1 and lib.d8s_bands_supported(9, 9, 51, 2) == 1
+    assert lib.d8s_bands_supported(18, 18, 39, 1) == 0            # 324 pixels
+    assert lib.d8s_bands_supported(18, 18, 39, 19) == 0           # more bands than rows
+    assert lib.d8s_bands_supported(9, 9, 65, 3) == 0              # more than 64 groups
+    assert lib.d8s_bands_supported(128, 128, 7, 128) == 1
+    assert lib.d8s_bands_supported(250, 125, 30, 125) == 0        # 2 rows of 125 pixels and their window: LDS
+    assert lib.d8s_bands_supported(9, 9, 51, 0) == 0 and lib.d8s_bands_supported(9, 9, 0, 1) == 0
+    lay = (hip.LayerP * 1)()
+    buf = (ctypes.c_uint8 * 64)()
+    p = ctypes.addressof(buf)
+    for h, w, bands, why in ((18, 18, 1, "256 pixels"), (18, 18, 19, "more bands"), (250, 125, 125, "LDS")):
+        args = hip.PartsArgs(p, p, ctypes.addressof(lay), p, p, 1, h, w, 2, 29, bands)
+        assert lib.d8s_dense_block_bands(ctypes.byref(args), None) == 1
+        assert why in lib.d8s_last_error().decode()
+
+
 def test_struct_layouts_match_header(tmp_path):
     prog = tmp_path / "layout.c"
     prog.write_text(

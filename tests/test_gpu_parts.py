@@ -136,6 +136,45 @@ def test_parts_wide_maps(dev, c4, kinds):
     assert torch.equal(got, c4["want"])
 
 
+@pytest.fixture(scope="module")
+def odd_maps(dev):
+    """Seeded DenseNets with short blocks at 288 px (maps 72, 36, 18, 9) and 416 px (104, 52, 26, 13): the
+    features with every layer as two launches."""
+    out = {}
+    for img, n in ((288, 3), (416, 2)):
+        model = densenet.seeded_densenet169(6, blocks=(2, 2, 4, 3)).to(dev)
+        x_u8 = synthetic.study_u8(n, img, seed=4)
+        cal = dense8s.calibrate(model, [synthetic.normalise(torch.from_numpy(x_u8).to(dev))])
+        pack = dense8s.make_pack(dense8s.make_plan(model.cpu(), cal, img), n, input_kind="u8")
+        x = torch.from_numpy(x_u8).to(dev)
+        out[img] = {"pack": pack, "x": x, "n": n,
+                    "want": dense8s.Dense8SEncoder(pack, dev.index or 0, n, fused={})(x).clone()}
+    return out
+
+
+@pytest.mark.parametrize("img,block,bands", [
+    (288, 2, 18), (416, 3, 13),                    # one pixel tile, partly filled (18 and 13 pixels)
+    (288, 1, 36), (288, 3, 2),                     # two (36 pixels; bands of 5 and 4 rows)
+    (288, 0, 72), (288, 2, 5), (288, 3, 1),        # up to four (72 pixels; uneven bands; one band, 81 pixels)
+    (416, 3, 3),                                   # 65 pixels: a tile of one pixel, bands of 5, 4 and 4 rows
+    (288, 0, 36), (416, 2, 4),                     # six (144 pixels; 182 in uneven bands)
+    (288, 0, 24), (416, 1, 13), (416, 0, 104)])    # eight (216, 208 pixels); 104-wide rows
+def test_bands_same_bytes(dev, odd_maps, img, block, bands):
+    """Bands of any row count and width (`d8s_dense_block_bands`): the bytes of two launches per layer,
+    eager and under graph replay, with no bounded wait running out."""
+    print(f"bands img={img} block={block} bands={bands}", flush=True)
+    m = odd_maps[img]
+    enc = dense8s.Dense8SEncoder(m["pack"], dev.index or 0, m["n"], fused={block: f"bands:{bands}"})
+    assert torch.equal(enc(m["x"]).clone(), m["want"])
+    enc.capture(m["n"])
+    for _ in range(2):
+        g = enc(m["x"]).clone()
+        _ = (m["x"].float() * 2).sum()
+        torch.cuda.synchronize(dev)
+        assert torch.equal(g, m["want"])
+    assert enc.sync_errors() == 0
+
+
 def test_parts_wait_error_surfaces(dev, c4):
     """A non-zero error word (planted by the host, as an expired wait would leave it) makes the pass's
     features NaN, reaches the host-mapped report, and makes the next call raise PartsWaitError, which
