@@ -118,3 +118,25 @@ def test_head_other_shapes(dev, d, w, slots, per, cd, targets, b):
     got = head.KneeHead(sd, dev, context_heads=cd // 64)(z.to(dev), slot_of, mask).cpu()
     assert got.shape == (b, targets)
     assert torch.allclose(got, want, rtol=1e-4, atol=1e-4), float((got - want).abs().max())
+
+
+@pytest.mark.parametrize("d,w,cd,targets,b", [
+    (64, 1, 64, 1, 1),               # one window, one finding, one k chunk
+    (130, 17, 192, 16, 2),           # a partial k group and chunk, two query groups, 32 dot columns
+    (1664, 65, 320, 12, 2),          # five heads: out_proj as its own product, h1 read from memory
+    (1664, 128, 256, 12, 5),         # several row tiles, the last partial; the longest study
+])
+def test_head_product_and_fusion_edges(dev, d, w, cd, targets, b):
+    """Edges of the product tiles, the k split and the two forms of out_proj, against the float32 oracle:
+    within 4e-6 of the largest logit (sums of up to 1664 products in float32 carry about 64 roundings of
+    2^-24 each, 4e-6 in all)."""
+    sd = H.random_state_dict(d + cd, d=d, slots=4, per=5, cd=cd, targets=targets)
+    g = torch.Generator().manual_seed(d)
+    z = torch.randn((b, w, d), generator=g) * 0.5
+    slot_of = torch.arange(w) % 4
+    mask = torch.rand((b, 4), generator=g) > 0.3
+    mask[0] = True
+    want = H.head_forward(sd, z, slot_of, mask, heads=cd // 64)
+    got = head.KneeHead(sd, dev, context_heads=cd // 64)(z.to(dev), slot_of, mask).cpu()
+    scale = want.abs().max().item()
+    assert (got - want).abs().max().item() <= 4e-6 * max(scale, 1.0)
