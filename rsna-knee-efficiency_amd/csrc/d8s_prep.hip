@@ -879,202 +879,297 @@ __global__ void __launch_bounds__(NT) k_prep_resize(PArgs a) {
 }
 
 // ---- grid sampling (geometric TTA view) -------------------------------------------------------
-// A thread owns one output pixel for a group of GIMG images: the grid is shared by all images, so the
-// source taps and weights are computed once and applied to each image (torch's grid_sampler_2d
-// arithmetic in float32, as its compiler contracts it, rounded once to fp16).  KIND 1 gathers the
-// images from the uint8 volume through the u / 255 fp16 table; KIND 2 is that gather alone.
+// A thread owns one output pixel, or four consecutive ones of a row, for a group of images: the grid is
+// shared by all images, so the source taps and weights are computed once and applied to each image
+// (torch's grid_sampler_2d arithmetic in float32, as its compiler contracts it, rounded once to fp16).
+// KIND 0 reads fp16 images, KIND 1 gathers uint8 slices through the u / 255 fp16 table.
 constexpr int GIMG = 8;
+
+// the source plane of image n (a slice index outside 0 .. SK-1 is clamped into it, so every read stays
+// inside the volume)
+template <int KIND>
+DEV int64_t grid_plane(const D8sGridArgs& a, int n) {
+    const int HW = a.H * a.W;
+    if constexpr (KIND == 1) {
+        const int b = n / a.M, m = n - b * a.M;
+        int64_t si = ((const int64_t*)a.slice_idx)[m];
+        si = si < 0 ? 0 : si >= a.SK ? (int64_t)a.SK - 1 : si;
+        return ((int64_t)b * a.SK + si) * HW;
+    } else {
+        return (int64_t)n * HW;
+    }
+}
+
+// Streaming stores: the output is not read back here, and kept out of the caches it leaves them to the
+// source rows the neighbouring blocks share (88 x 3 windows of 512 x 512: 100 -> 83 us).
+DEV void nt_store64(void* p, uint32_t lo, uint32_t hi) {
+    __builtin_nontemporal_store((uint64_t)lo | (uint64_t)hi << 32, (uint64_t*)p);
+}
+
+// Taps (nw, ne, sw, se), weights and which taps lie inside the image, of one output pixel.
+struct Tap {
+    int x0, y0;
+    float w[4];
+    bool ok[4];
+};
+
+DEV Tap grid_tap(const D8sGridArgs& a, uint32_t gbits) {
+    Tap t;
+    const __half2 g = __builtin_bit_cast(__half2, gbits);
+    const float gx = __low2float(g), gy = __high2float(g);
+    const float ix = __builtin_fmaf(gx + 1.0f, (float)a.W, -1.0f) * 0.5f;
+    const float iy = __builtin_fmaf(gy + 1.0f, (float)a.H, -1.0f) * 0.5f;
+    t.x0 = (int)floorf(ix);
+    t.y0 = (int)floorf(iy);
+    const int x1 = t.x0 + 1, y1 = t.y0 + 1;
+    t.w[0] = ((float)x1 - ix) * ((float)y1 - iy);
+    t.w[1] = (ix - (float)t.x0) * ((float)y1 - iy);
+    t.w[2] = ((float)x1 - ix) * (iy - (float)t.y0);
+    t.w[3] = (ix - (float)t.x0) * (iy - (float)t.y0);
+    const bool vx0 = t.x0 >= 0 && t.x0 < a.W, vx1 = x1 >= 0 && x1 < a.W;
+    const bool vy0 = t.y0 >= 0 && t.y0 < a.H, vy1 = y1 >= 0 && y1 < a.H;
+    t.ok[0] = vy0 && vx0;
+    t.ok[1] = vy0 && vx1;
+    t.ok[2] = vy1 && vx0;
+    t.ok[3] = vy1 && vx1;
+    return t;
+}
+
+// One pixel of NI images: every gather of every image issued before the first is used (taps outside the
+// image read the plane's first pixel and are not added).  lut(u): the float32 value of byte u.
+template <int KIND, int NI, class L>
+DEV void grid_pixel(const D8sGridArgs& a, const Tap& t, const int64_t (&pl)[NI], float (&acc)[NI], L&& lut) {
+    const int off[4] = {t.ok[0] ? t.y0 * a.W + t.x0 : 0, t.ok[1] ? t.y0 * a.W + t.x0 + 1 : 0,
+                        t.ok[2] ? (t.y0 + 1) * a.W + t.x0 : 0, t.ok[3] ? (t.y0 + 1) * a.W + t.x0 + 1 : 0};
+    uint16_t v[NI][4];
+#pragma unroll
+    for (int i = 0; i < NI; ++i)
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            if constexpr (KIND == 1)
+                v[i][k] = ((const uint8_t*)a.src)[pl[i] + off[k]];
+            else
+                v[i][k] = ((const uint16_t*)a.src)[pl[i] + off[k]];
+        }
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+        acc[i] = 0.0f;
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+            if (t.ok[k]) acc[i] = __builtin_fmaf(KIND == 1 ? lut(v[i][k]) : __half2float(__ushort_as_half(v[i][k])), t.w[k], acc[i]);
+    }
+}
 
 template <int KIND>
 __global__ void __launch_bounds__(NT) k_grid_sample(D8sGridArgs a) {
     __shared__ uint16_t s_lut[256];
-    if constexpr (KIND >= 1) {
-        if (threadIdx.x < 256) s_lut[threadIdx.x] = ((const uint16_t*)a.lut)[threadIdx.x];
+    if constexpr (KIND == 1) {
+        s_lut[threadIdx.x] = ((const uint16_t*)a.lut)[threadIdx.x];
         __syncthreads();
     }
     const int HW = a.H * a.W;
     const int p = blockIdx.x * NT + threadIdx.x;
     const int n0 = blockIdx.y * GIMG, n1 = min(n0 + GIMG, a.N);
     if (p >= HW) return;
-    // the image n: its source plane
-    // (a slice index outside 0 .. SK-1 is clamped into it, so every read stays inside the volume)
-    auto plane = [&](int n) -> int64_t {
-        if constexpr (KIND >= 1) {
-            const int b = n / a.M, m = n - b * a.M;
-            int64_t si = ((const int64_t*)a.slice_idx)[m];
-            si = si < 0 ? 0 : si >= a.SK ? (int64_t)a.SK - 1 : si;
-            return ((int64_t)b * a.SK + si) * HW;
-        } else {
-            return (int64_t)n * HW;
-        }
-    };
-    // the GIMG images' planes first (their slice indices are loads), then every gather of every image
-    // (loads clamped to the last image, stores predicated), so they are all in flight together
     int64_t pl[GIMG];
 #pragma unroll
-    for (int i = 0; i < GIMG; ++i) pl[i] = plane(min(n0 + i, n1 - 1));
-    if constexpr (KIND == 2) {
-        uint8_t v[GIMG];
+    for (int i = 0; i < GIMG; ++i) pl[i] = grid_plane<KIND>(a, min(n0 + i, n1 - 1));
+    const Tap t = grid_tap(a, ((const uint32_t*)a.grid)[p]);
+    float acc[GIMG];
+    grid_pixel<KIND, GIMG>(a, t, pl, acc, [&](uint32_t u) { return __half2float(__ushort_as_half(s_lut[u])); });
 #pragma unroll
-        for (int i = 0; i < GIMG; ++i) v[i] = ((const uint8_t*)a.src)[pl[i] + p];
+    for (int i = 0; i < GIMG; ++i)
+        if (n0 + i < n1) ((__half*)a.out)[(int64_t)(n0 + i) * HW + p] = __float2half_rn(acc[i]);
+}
+
+// The gather alone (no grid): out = lut[slice], 8 consecutive pixels of a plane per thread (the last of a
+// plane that is no multiple of 8 takes its pixels singly).  Planes of any size and address: the loads and
+// stores are 8 bytes at byte (2-byte) alignment, which the hardware takes.  The table in 16 copies, a
+// lane's by its index, keeps random bytes off one bank; 88 x 3 windows of 512 x 512: 131 -> 57 us (a byte
+// and a 2-byte store a thread and image before), of 449 x 449 115 -> 62.
+struct __attribute__((packed)) u64_any { uint64_t v; };
+__global__ void __launch_bounds__(NT) k_grid_gather(D8sGridArgs a) {
+    constexpr int GC = 16;
+    __shared__ __attribute__((aligned(16))) uint32_t s_lut[256 * GC];
+    {
+        const uint32_t x = ((const uint16_t*)a.lut)[threadIdx.x];
 #pragma unroll
-        for (int i = 0; i < GIMG; ++i)
-            if (n0 + i < n1) ((uint16_t*)a.out)[(int64_t)(n0 + i) * HW + p] = s_lut[v[i]];
+        for (int c = 0; c < GC; c += 4) *(uint4*)&s_lut[threadIdx.x * GC + c] = make_uint4(x, x, x, x);
+    }
+    __syncthreads();
+    const uint32_t lc = threadIdx.x % GC;
+    const int HW = a.H * a.W;
+    const int64_t p = 8 * ((int64_t)blockIdx.x * NT + threadIdx.x);
+    const int n0 = blockIdx.y * GIMG, n1 = min(n0 + GIMG, a.N);
+    if (p >= HW) return;
+    const uint8_t* src = (const uint8_t*)a.src;
+    if (p + 8 > HW) {
+        for (int n = n0; n < n1; ++n) {
+            const int64_t pl = grid_plane<1>(a, n);
+            for (int64_t q = p; q < HW; ++q) ((uint16_t*)a.out)[(int64_t)n * HW + q] = (uint16_t)s_lut[src[pl + q] * GC + lc];
+        }
         return;
-    } else {
-        const __half2 g = ((const __half2*)a.grid)[p];
-        const float gx = __low2float(g), gy = __high2float(g);
-        const float ix = __builtin_fmaf(gx + 1.0f, (float)a.W, -1.0f) * 0.5f;
-        const float iy = __builtin_fmaf(gy + 1.0f, (float)a.H, -1.0f) * 0.5f;
-        const int x0 = (int)floorf(ix), y0 = (int)floorf(iy);
-        const int x1 = x0 + 1, y1 = y0 + 1;
-        const float w[4] = {((float)x1 - ix) * ((float)y1 - iy), (ix - (float)x0) * ((float)y1 - iy),
-                            ((float)x1 - ix) * (iy - (float)y0), (ix - (float)x0) * (iy - (float)y0)};
-        const bool vx0 = x0 >= 0 && x0 < a.W, vx1 = x1 >= 0 && x1 < a.W;
-        const bool vy0 = y0 >= 0 && y0 < a.H, vy1 = y1 >= 0 && y1 < a.H;
-        const bool ok[4] = {vy0 && vx0, vy0 && vx1, vy1 && vx0, vy1 && vx1};
-        // taps outside the image read the plane's first pixel and are not added
-        const int off[4] = {ok[0] ? y0 * a.W + x0 : 0, ok[1] ? y0 * a.W + x1 : 0,
-                            ok[2] ? y1 * a.W + x0 : 0, ok[3] ? y1 * a.W + x1 : 0};
-        float v[GIMG][4];
+    }
+    int64_t pl[GIMG];
 #pragma unroll
-        for (int i = 0; i < GIMG; ++i)
+    for (int i = 0; i < GIMG; ++i) pl[i] = grid_plane<1>(a, min(n0 + i, n1 - 1));
+    uint64_t v[GIMG];
 #pragma unroll
-            for (int t = 0; t < 4; ++t) {
-                if constexpr (KIND == 1)
-                    v[i][t] = (float)((const uint8_t*)a.src)[pl[i] + off[t]];
-                else
-                    v[i][t] = __half2float(((const __half*)a.src)[pl[i] + off[t]]);
-            }
+    for (int i = 0; i < GIMG; ++i) v[i] = ((const u64_any*)(src + pl[i] + p))->v;
 #pragma unroll
-        for (int i = 0; i < GIMG; ++i) {
-            float acc = 0.0f;
+    for (int i = 0; i < GIMG; ++i) {
+        if (n0 + i >= n1) break;
+        uint16_t* out = (uint16_t*)a.out + (int64_t)(n0 + i) * HW + p;
+        uint32_t o[4];
 #pragma unroll
-            for (int t = 0; t < 4; ++t) {
-                if (ok[t]) {
-                    float x = v[i][t];
-                    if constexpr (KIND == 1) x = __half2float(__ushort_as_half(s_lut[(int)x]));
-                    acc = __builtin_fmaf(x, w[t], acc);
-                }
-            }
-            if (n0 + i < n1) ((__half*)a.out)[(int64_t)(n0 + i) * HW + p] = __float2half_rn(acc);
+        for (int k = 0; k < 4; ++k) {
+            const uint32_t w = (uint32_t)(v[i] >> (16 * k));
+            o[k] = s_lut[(w & 0xffu) * GC + lc] | (s_lut[((w >> 8) & 0xffu) * GC + lc] << 16);
+        }
+        if (((uintptr_t)out & 7) == 0) {
+            nt_store64(out, o[0], o[1]);
+            nt_store64(out + 4, o[2], o[3]);
+        } else {
+            ((u64_any*)out)->v = (uint64_t)o[0] | (uint64_t)o[1] << 32;
+            ((u64_any*)(out + 4))->v = (uint64_t)o[2] | (uint64_t)o[3] << 32;
         }
     }
 }
 
-// The uint8 gather + table + bilinear view (KIND 1 above) with four consecutive output pixels of a row
-// per thread (W a multiple of 4, the grid 16-byte aligned).  Where the four pixels share their source
-// rows and all their taps lie in one 8-byte aligned window of those rows inside the image (a zoom or
-// shift of at most about 1.75 source pixels per output pixel), each image's taps come from two dword
-// loads per row instead of sixteen byte loads; elsewhere each pixel takes KIND 1's taps.  Per pixel the
-// arithmetic is KIND 1's (the same values, weights and fma order), so the outputs are identical.
-// GIMG4 images per thread (16 measured 8 % faster than 8 and than 4 at the submission's shape).
-constexpr int GIMG4 = 16;
+// Four consecutive output pixels of a row per thread (W a multiple of 4, the grid 16-byte aligned).  Where
+// the four share their two source rows inside the image and their left taps advance by at most one column
+// a pixel (a zoom in, a shift: o_k in {k - 1, k} from the first's), or by at least one (a zoom out of less
+// than a third: {k, k + 1}), their taps are at most 5 (6) columns of the two rows: two dwords (KIND 0: 16
+// bytes) per row and image, each column converted once, a pixel's two picked by one select a row.
+// Elsewhere each pixel takes the one-pixel kernel's taps.  Per pixel the values, weights and fma order are
+// the one-pixel kernel's, so the outputs are identical.  What bounded the uint8 form was the table in LDS:
+// sixteen lookups of random entries a thread and image, about four lanes on one bank each; now ten (twelve)
+// in a table of NC float32 copies, a lane's
+// copy by its index, and streaming stores (88 x 3 windows of 512 x 512: 101 -> 82 us, zoomed out 180 -> 148;
+// fp16 images, which had one pixel a thread, 92 -> 50).  The grid's x blocks are renumbered so
+// that each XCD's share is consecutive rows (neighbouring blocks read the same source rows: one L2).
+constexpr int NC = 16;
+template <int KIND>
+constexpr int G4IMG = KIND == 1 ? 4 : 8;     // images per thread
+
+template <int KIND>
 __global__ void __launch_bounds__(NT) k_grid_sample4(D8sGridArgs a) {
-    __shared__ uint16_t s_lut[256];
-    if (threadIdx.x < 256) s_lut[threadIdx.x] = ((const uint16_t*)a.lut)[threadIdx.x];
-    __syncthreads();
+    constexpr int NI = G4IMG<KIND>;
+    __shared__ __attribute__((aligned(16))) float s_lut[KIND == 1 ? 256 * NC : 4];
+    if constexpr (KIND == 1) {
+        const float x = __half2float(__ushort_as_half(((const uint16_t*)a.lut)[threadIdx.x]));
+#pragma unroll
+        for (int c = 0; c < NC; c += 4) *(float4*)&s_lut[threadIdx.x * NC + c] = make_float4(x, x, x, x);
+        __syncthreads();
+    }
     const int HW = a.H * a.W;
-    const int p0 = 4 * (blockIdx.x * NT + threadIdx.x);
-    const int n0 = blockIdx.y * GIMG4, n1 = min(n0 + GIMG4, a.N);
+    const int per = (int)gridDim.x / 8;                       // (gridDim.x is a multiple of 8)
+    const int p0 = 4 * ((((int)blockIdx.x % 8) * per + (int)blockIdx.x / 8) * NT + (int)threadIdx.x);
+    const int n0 = blockIdx.y * NI, n1 = min(n0 + NI, a.N);
     if (p0 >= HW) return;
-    int64_t pl[GIMG4];
+    int64_t pl[NI];
 #pragma unroll
-    for (int i = 0; i < GIMG4; ++i) {
-        const int n = min(n0 + i, n1 - 1), b = n / a.M, m = n - b * a.M;
-        int64_t si = ((const int64_t*)a.slice_idx)[m];
-        si = si < 0 ? 0 : si >= a.SK ? (int64_t)a.SK - 1 : si;
-        pl[i] = ((int64_t)b * a.SK + si) * HW;
-    }
+    for (int i = 0; i < NI; ++i) pl[i] = grid_plane<KIND>(a, min(n0 + i, n1 - 1));
     const uint4 gq = ((const uint4*)a.grid)[p0 >> 2];         // 4 pixels x (gx, gy) fp16
-    const uint32_t gw[4] = {gq.x, gq.y, gq.z, gq.w};
-    float w[4][4];
-    int x0[4], y0[4];
-    bool ok[4][4];
+    const Tap t[4] = {grid_tap(a, gq.x), grid_tap(a, gq.y), grid_tap(a, gq.z), grid_tap(a, gq.w)};
+    const uint32_t lane_off = (threadIdx.x % NC) * 4;
+    auto lut = [&](uint32_t at) {                             // at = 4 NC u
+        return *(const float*)((const char*)s_lut + (at | lane_off));
+    };
+    const int x0 = t[0].x0, y0 = t[0].y0;
+    constexpr int AL = KIND == 1 ? 4 : 2;                     // pixels per dword
+    const int base = x0 & ~(AL - 1);
+    const bool rows = t[1].y0 == y0 && t[2].y0 == y0 && t[3].y0 == y0 && y0 >= 0 && y0 < a.H - 1 && x0 >= 0 && base <= a.W - 8;
+    bool in = rows, out = rows;
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-        const __half2 g = __builtin_bit_cast(__half2, gw[k]);
-        const float gx = __low2float(g), gy = __high2float(g);
-        const float ix = __builtin_fmaf(gx + 1.0f, (float)a.W, -1.0f) * 0.5f;
-        const float iy = __builtin_fmaf(gy + 1.0f, (float)a.H, -1.0f) * 0.5f;
-        x0[k] = (int)floorf(ix);
-        y0[k] = (int)floorf(iy);
-        const int x1 = x0[k] + 1, y1 = y0[k] + 1;
-        w[k][0] = ((float)x1 - ix) * ((float)y1 - iy);
-        w[k][1] = (ix - (float)x0[k]) * ((float)y1 - iy);
-        w[k][2] = ((float)x1 - ix) * (iy - (float)y0[k]);
-        w[k][3] = (ix - (float)x0[k]) * (iy - (float)y0[k]);
-        const bool vx0 = x0[k] >= 0 && x0[k] < a.W, vx1 = x1 >= 0 && x1 < a.W;
-        const bool vy0 = y0[k] >= 0 && y0[k] < a.H, vy1 = y1 >= 0 && y1 < a.H;
-        ok[k][0] = vy0 && vx0;
-        ok[k][1] = vy0 && vx1;
-        ok[k][2] = vy1 && vx0;
-        ok[k][3] = vy1 && vx1;
+    for (int k = 1; k < 4; ++k) {
+        const int o = t[k].x0 - x0;
+        in &= o == k - 1 || o == k;
+        out &= o == k || o == k + 1;
     }
-    const int xmin = min(min(x0[0], x0[1]), min(x0[2], x0[3])), xmax = max(max(x0[0], x0[1]), max(x0[2], x0[3]));
-    const int base = xmin & ~3;
-    const bool fast = y0[0] == y0[1] && y0[0] == y0[2] && y0[0] == y0[3] && y0[0] >= 0 && y0[0] + 1 < a.H &&
-                      xmin >= 0 && xmax + 1 - base <= 7 && base + 8 <= a.W;
-    float acc[GIMG4][4];
-    if (fast) {
-        // rows y0, y0 + 1 of each image: bytes base .. base + 7 as two dwords per row
-        const int r0 = y0[0] * a.W + base;
-        uint32_t d[GIMG4][4];
+    // (a zoom out's columns x0 .. x0 + 5 may reach into a third dword of bytes)
+    out &= KIND == 0 || base <= a.W - 12;
+    float acc[NI][4];
+    // SH: pixel k's left column is k - 1 + SH or k + SH
+    auto fast = [&](auto sh) __attribute__((always_inline)) {
+        constexpr int SH = decltype(sh)::value, COLS = 5 + SH;
+        const int r0 = y0 * a.W + base;
+        constexpr int DW = KIND == 1 ? 2 + SH : 4;
+        uint32_t d[NI][2][DW];
 #pragma unroll
-        for (int i = 0; i < GIMG4; ++i) {
-            const uint32_t* q0 = (const uint32_t*)((const uint8_t*)a.src + pl[i] + r0);
-            const uint32_t* q1 = (const uint32_t*)((const uint8_t*)a.src + pl[i] + r0 + a.W);
-            d[i][0] = q0[0];
-            d[i][1] = q0[1];
-            d[i][2] = q1[0];
-            d[i][3] = q1[1];
-        }
+        for (int i = 0; i < NI; ++i)
 #pragma unroll
-        for (int i = 0; i < GIMG4; ++i) {
-            const uint64_t row0 = (uint64_t)d[i][0] | ((uint64_t)d[i][1] << 32);
-            const uint64_t row1 = (uint64_t)d[i][2] | ((uint64_t)d[i][3] << 32);
+            for (int r = 0; r < 2; ++r) {
+                const uint32_t* q = (const uint32_t*)((const uint8_t*)a.src + (KIND == 1 ? 1 : 2) * (pl[i] + r0 + r * a.W));
+#pragma unroll
+                for (int w = 0; w < DW; ++w) d[i][r][w] = q[w];
+            }
+        const uint32_t sft = (uint32_t)(x0 - base) * (KIND == 1 ? 8 : 16);
+        bool up[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) up[k] = t[k].x0 - x0 == k + SH;
+#pragma unroll
+        for (int i = 0; i < NI; ++i) {
+            float c[2][COLS + (COLS & 1)];
+#pragma unroll
+            for (int r = 0; r < 2; ++r) {
+                if constexpr (KIND == 1) {
+                    const uint32_t lo = __builtin_amdgcn_alignbit(d[i][r][1], d[i][r][0], sft);
+                    const uint32_t hi = __builtin_amdgcn_alignbit(d[i][r][DW - 1], d[i][r][1], sft);
+                    constexpr uint32_t M = 255u * 4 * NC;
+                    static_assert(NC == 16, "byte u at bit 6: 4 NC u");
+                    c[r][0] = lut((lo << 6) & M);
+                    c[r][1] = lut((lo >> 2) & M);
+                    c[r][2] = lut((lo >> 10) & M);
+                    c[r][3] = lut((lo >> 18) & M);
+                    c[r][4] = lut((hi << 6) & M);
+                    if constexpr (COLS > 5) c[r][5] = lut((hi >> 2) & M);
+                } else {
+#pragma unroll
+                    for (int w = 0; w < 3; ++w) {
+                        const __half2 v = __builtin_bit_cast(__half2, __builtin_amdgcn_alignbit(d[i][r][w + 1], d[i][r][w], sft));
+                        c[r][2 * w] = __low2float(v);
+                        if (2 * w + 1 < COLS) c[r][2 * w + 1] = __high2float(v);
+                    }
+                }
+            }
 #pragma unroll
             for (int k = 0; k < 4; ++k) {
-                const int o = 8 * (x0[k] - base);
-                const uint32_t t0 = (uint32_t)(row0 >> o), t1 = (uint32_t)(row1 >> o);
-                const float v[4] = {__half2float(__ushort_as_half(s_lut[t0 & 0xffu])),
-                                    __half2float(__ushort_as_half(s_lut[(t0 >> 8) & 0xffu])),
-                                    __half2float(__ushort_as_half(s_lut[t1 & 0xffu])),
-                                    __half2float(__ushort_as_half(s_lut[(t1 >> 8) & 0xffu]))};
                 float s = 0.0f;
 #pragma unroll
-                for (int t = 0; t < 4; ++t) s = __builtin_fmaf(v[t], w[k][t], s);
+                for (int r = 0; r < 2; ++r) {
+                    // (pixel 0 of a zoom in has o = 0: column 0; of a zoom out 0 too)
+                    const int lo = k - 1 + SH;
+                    const float l = lo < 0 || (SH == 1 && k == 0) ? c[r][0] : up[k] ? c[r][lo + 1] : c[r][lo];
+                    const float h = lo < 0 || (SH == 1 && k == 0) ? c[r][1] : up[k] ? c[r][lo + 2] : c[r][lo + 1];
+                    s = __builtin_fmaf(l, t[k].w[2 * r], s);
+                    s = __builtin_fmaf(h, t[k].w[2 * r + 1], s);
+                }
                 acc[i][k] = s;
             }
         }
+    };
+    if (in) {
+        fast(std::integral_constant<int, 0>{});
+    } else if (out) {
+        fast(std::integral_constant<int, 1>{});
     } else {
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
-            const int off[4] = {ok[k][0] ? y0[k] * a.W + x0[k] : 0, ok[k][1] ? y0[k] * a.W + x0[k] + 1 : 0,
-                                ok[k][2] ? (y0[k] + 1) * a.W + x0[k] : 0, ok[k][3] ? (y0[k] + 1) * a.W + x0[k] + 1 : 0};
-            float v[GIMG4][4];
+            float v[NI];
+            grid_pixel<KIND, NI>(a, t[k], pl, v, [&](uint32_t u) { return lut(u * 4 * NC); });
 #pragma unroll
-            for (int i = 0; i < GIMG4; ++i)
-#pragma unroll
-                for (int t = 0; t < 4; ++t) v[i][t] = (float)((const uint8_t*)a.src)[pl[i] + off[t]];
-#pragma unroll
-            for (int i = 0; i < GIMG4; ++i) {
-                float s = 0.0f;
-#pragma unroll
-                for (int t = 0; t < 4; ++t)
-                    if (ok[k][t]) s = __builtin_fmaf(__half2float(__ushort_as_half(s_lut[(int)v[i][t]])), w[k][t], s);
-                acc[i][k] = s;
-            }
+            for (int i = 0; i < NI; ++i) acc[i][k] = v[i];
         }
     }
 #pragma unroll
-    for (int i = 0; i < GIMG4; ++i)
+    for (int i = 0; i < NI; ++i)
         if (n0 + i < n1) {
             const uint32_t lo = (uint32_t)__half_as_ushort(__float2half_rn(acc[i][0])) |
                                 ((uint32_t)__half_as_ushort(__float2half_rn(acc[i][1])) << 16);
             const uint32_t hi = (uint32_t)__half_as_ushort(__float2half_rn(acc[i][2])) |
                                 ((uint32_t)__half_as_ushort(__float2half_rn(acc[i][3])) << 16);
-            *(uint2*)((uint16_t*)a.out + (int64_t)(n0 + i) * HW + p0) = make_uint2(lo, hi);
+            nt_store64((uint16_t*)a.out + (int64_t)(n0 + i) * HW + p0, lo, hi);
         }
 }
 
@@ -1326,16 +1421,23 @@ extern "C" int d8s_grid_sample(const D8sGridArgs* a, void* stream) {
         PREQ((int64_t)a->B * a->M == a->N, "N must be B * M");
     }
     PREQ(a->N >= 1 && a->N < 65536 * GIMG, "N must be 1 .. 524287");
-    const dim3 grid((unsigned)(((int64_t)a->H * a->W + NT - 1) / NT), (unsigned)((a->N + GIMG - 1) / GIMG));
+    const int64_t HW = (int64_t)a->H * a->W;
+    const dim3 grid((unsigned)((HW + NT - 1) / NT), (unsigned)((a->N + GIMG - 1) / GIMG));
     hipStream_t st = (hipStream_t)stream;
-    if (a->kind == 1 && a->grid != 0 && a->W % 4 == 0 && a->grid % 16 == 0 && a->out % 8 == 0 && a->src % 4 == 0) {
-        const dim3 grid4((unsigned)(((int64_t)a->H * a->W / 4 + NT - 1) / NT), (unsigned)((a->N + GIMG4 - 1) / GIMG4));
-        k_grid_sample4<<<grid4, NT, 0, st>>>(*a);
-    } else if (a->kind == 1 && a->grid == 0)
-        k_grid_sample<2><<<grid, NT, 0, st>>>(*a);
-    else if (a->kind == 1)
+    if (a->grid == 0) {
+        k_grid_gather<<<dim3((unsigned)((HW + 8 * NT - 1) / (8 * NT)), grid.y), NT, 0, st>>>(*a);
+    } else if (a->W % 4 == 0 && a->grid % 16 == 0 && a->out % 8 == 0 && a->src % 4 == 0) {
+        // four pixels a thread: rows of whole dwords (uint8 and fp16 alike), the grid's and output's quads
+        // aligned
+        const unsigned gx = (unsigned)((HW / 4 + NT - 1) / NT + 7) / 8 * 8;
+        if (a->kind == 1)
+            k_grid_sample4<1><<<dim3(gx, (unsigned)((a->N + G4IMG<1> - 1) / G4IMG<1>)), NT, 0, st>>>(*a);
+        else
+            k_grid_sample4<0><<<dim3(gx, (unsigned)((a->N + G4IMG<0> - 1) / G4IMG<0>)), NT, 0, st>>>(*a);
+    } else if (a->kind == 1) {
         k_grid_sample<1><<<grid, NT, 0, st>>>(*a);
-    else
+    } else {
         k_grid_sample<0><<<grid, NT, 0, st>>>(*a);
+    }
     return d8s_host_launched("d8s_grid_sample");
 }

@@ -128,3 +128,39 @@ def test_windows_u8_slice_checks(dev, view):
     ref = torch.empty_like(out2)
     tta.windows_u8(v, clamped, ref, *view)
     assert torch.equal(out2, ref)
+
+
+@pytest.mark.parametrize("kind", [0, 1])
+@pytest.mark.parametrize("h,w,off", [(5, 4, 0), (7, 8, 0), (9, 12, 0), (33, 64, 0), (33, 64, 1), (20, 61, 0), (3, 3, 1)])
+@pytest.mark.parametrize("view", [(1.0, 0.0, 0.0), (1.5, 0.0, 0.0), (1.25, 0.11, -0.2), (0.8, 0.0, 0.05), (0.6, 0.0, 0.0),
+                                  (1.0, 0.02, 0.0)])
+def test_grid_sample_kernels_agree(dev, kind, h, w, off, view):
+    """The four-pixel form's three paths (zoom in, zoom out, borders), narrow and odd images, images that
+    start at an odd element (`off`: the one-pixel form, the gather's unaligned loads) and group remainders,
+    through the C ABI: bit for bit torch's grid_sample (the table alone for the identity) on the same
+    values, and nothing written around the output."""
+    import ctypes
+    from rsna_knee_efficiency_amd import hip
+    if kind == 0 and view == (1.0, 0.0, 0.0):
+        pytest.skip("fp16 images have no gather")
+    n, sk = 19, 5
+    print(f"grid kind={kind} {h}x{w} off={off} view={view}", flush=True)
+    g = torch.Generator().manual_seed(h * w + off)
+    lut = tta.lut_u8_f16(dev)
+    idx = torch.randint(0, sk, (n,), generator=g).to(dev)
+    if kind == 1:
+        buf = torch.randint(0, 256, (off + sk * h * w,), generator=g, dtype=torch.uint8).to(dev)
+        imgs = lut[buf[off:].view(sk, h, w)[idx].long()]
+    else:
+        buf = torch.rand((off + n * h * w,), generator=g).half().to(dev)
+        imgs = buf[off:].view(n, h, w)
+    out = torch.full((8 + n * h * w + 8,), 9.0, dtype=torch.float16, device=dev)
+    grid = None if view == (1.0, 0.0, 0.0) else tta.view_grid(h, w, 1, *view, torch.float16, dev)
+    a = hip.GridArgs(src=buf.data_ptr() + off * buf.element_size(), slice_idx=idx.data_ptr(), lut=lut.data_ptr(),
+                     grid=0 if grid is None else grid.data_ptr(), out=out.data_ptr() + 16, kind=kind, N=n, H=h, W=w,
+                     B=1, SK=sk, M=n)
+    hip.call("d8s_grid_sample", ctypes.byref(a), ctypes.c_void_p(torch.cuda.current_stream(dev).cuda_stream))
+    want = imgs if grid is None else F.grid_sample(imgs.contiguous()[:, None], grid.expand(n, h, w, 2), mode="bilinear",
+                                                   padding_mode="zeros", align_corners=False)[:, 0]
+    assert torch.equal(out[8:-8].view(n, h, w), want)
+    assert bool((out[:8] == 9).all()) and bool((out[-8:] == 9).all())
