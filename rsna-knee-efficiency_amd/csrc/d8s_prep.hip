@@ -36,6 +36,7 @@
 #include <math.h>
 #include <stdint.h>
 
+#include <algorithm>
 #include <string>
 #include <type_traits>
 
@@ -94,7 +95,7 @@ struct PStack {
     int ns_max, rp, dpl; // source rows a block may read; LDS dwords per staged raw row; per lane
     int dbuf;            // 1: two raw buffers (block b+1 copied during block b's x pass); 0: one
     float inv_rp;
-    int hb, hb2, nb;     // blocks per workgroup: histogram level 1, levels 2-3, final pass
+    int hb, hb2, nb;     // blocks per workgroup: level 1 of regions, float32 levels, final pass
     int wg_hist, wg_hist2, wg_norm;  // first workgroup of this stack in each grid
 };
 
@@ -257,11 +258,11 @@ DEV float rescale(uint32_t u, float sl, float ic) {
 // The area taps of an output index are consecutive source indices (raw_crop.py:361-369), so a tap's
 // source is the first index + t; a zero-weight padding tap then reads a neighbour instead of index 0,
 // which changes nothing for finite values (x * 0 = +-0 added to a sum that is never -0).
-template <int MODE, bool HAS, bool WROW, class F>
+template <int MODE, bool HAS, bool WROW, int TH = NT, class F>
 DEV void run_blocks(const PStack& st, const PArgs& a, int b0, int b1, float* s_st, F&& f) {
     const int img = a.img;
     if constexpr (MODE == M_FLOAT) {
-        // a thread's units u = tid + NT i of a block in batches of FB: the batch's loads are issued
+        // a thread's units u = tid + TH i of a block in batches of FB: the batch's loads are issued
         // before any of its values is used (the histogram passes' LDS atomics would otherwise keep
         // each load behind the previous unit's counting); units past the block load its last unit
         // again and are not used
@@ -270,12 +271,12 @@ DEV void run_blocks(const PStack& st, const PArgs& a, int b0, int b1, float* s_s
             const Geo g = block_geo<MODE>(st, a, b);
             const int n = g.rb * a.upr;
             const float* base = (const float*)st.src + (int64_t)g.kk * img * img;
-            for (int u0 = threadIdx.x; u0 < n; u0 += FB * NT) {
+            for (int u0 = threadIdx.x; u0 < n; u0 += FB * TH) {
                 float4 x[FB];
                 int dy[FB], dx0[FB];
 #pragma unroll
                 for (int i = 0; i < FB; ++i) {
-                    const int u = min(u0 + i * NT, n - 1);
+                    const int u = min(u0 + i * TH, n - 1);
                     const int row = fdiv(u, a.upr, a.inv_upr);
                     dx0[i] = (u - row * a.upr) * UP;
                     dy[i] = g.r0 + row;
@@ -283,7 +284,7 @@ DEV void run_blocks(const PStack& st, const PArgs& a, int b0, int b1, float* s_s
                 }
 #pragma unroll
                 for (int i = 0; i < FB; ++i) {
-                    if (u0 + i * NT < n) {
+                    if (u0 + i * TH < n) {
                         float v[UP] = {x[i].x, x[i].y, x[i].z, x[i].w};
                         f(g.kk, dy[i], dx0[i], v);
                     }
@@ -542,7 +543,7 @@ DEV void with_mode(const PStack& st, const PArgs& a, B&& body) {
     }
 }
 
-// grid 0: histogram level 1; 1: levels 2 and 3; 2: final pass and resize
+// grid 0: histogram level 1 of regions; 1: the float32 levels; 2: final pass and resize
 DEV int first_wg(const PStack& p, int grid) { return grid == 0 ? p.wg_hist : grid == 1 ? p.wg_hist2 : p.wg_norm; }
 
 DEV int stack_of(const PArgs& a, int grid) {
@@ -593,16 +594,26 @@ __global__ void __launch_bounds__(NT) k_prep_setup(PArgs a, int clear) {
     }
 }
 
-// One radix level over the blocks [b0, b0 + hb) of one stack.
+// One radix level over the blocks [b0, b0 + hb) of one stack.  Float32 stacks run wide workgroups over
+// many blocks (wide_view): noisy values fill most of a level-2 histogram, and each workgroup adds its
+// nonzero bins to the global one, so their number is what that costs (level 2 of 8 stacks of 24 x 288^2:
+// 25 us with 1012 workgroups of 256, 21 with 506 of 1024).
+constexpr int WIDE = 1024;
 template <int LEVEL, int REGION, bool STORE = false>
-__global__ void __launch_bounds__(NT) k_prep_hist(PArgs a) {
+__global__ void __launch_bounds__(LEVEL == 1 && REGION ? NT : WIDE) k_prep_hist(PArgs a) {
+    constexpr bool WD = LEVEL > 1 || !REGION;
+    constexpr int TH = WD ? WIDE : NT;
+    // level 1 of float32 stacks: copies of its histogram, a lane's by its index.  The keys' top bits put
+    // neighbouring values in few bins, so 64 lanes adding to one copy would mostly wait for each other
+    // (and runs kept per thread broke at almost every unit of noisy values: 22.5 us, now 19.3)
+    constexpr int CP = LEVEL == 1 && !REGION ? 8 : 1;
     constexpr int NB = LEVEL == 1 ? NB1 : LEVEL == 2 ? NB2 : NB3;
     constexpr int NH = LEVEL == 1 ? 1 : 2;    // LDS histograms; slots 2 and 3 (rare) count in memory
-    __shared__ uint32_t s_h[NH * NB];
+    __shared__ uint32_t s_h[NH * NB * CP];
     __shared__ float s_st[REGION ? STAGE : 1];
-    const int s = stack_of(a, LEVEL == 1 ? 0 : 1);
+    const int s = stack_of(a, WD ? 1 : 0);
     const PStack& st = a.s[s];
-    for (int i = threadIdx.x; i < NH * NB; i += NT) s_h[i] = 0u;
+    for (int i = threadIdx.x; i < NH * NB * CP; i += TH) s_h[i] = 0u;
     uint32_t nslot = 0, pre[4] = {0u, 0u, 0u, 0u};
     if constexpr (LEVEL > 1) {
         const Sel* sel = (const Sel*)(st.ws + (LEVEL == 2 ? W_SEL1 : W_SEL2));
@@ -611,8 +622,8 @@ __global__ void __launch_bounds__(NT) k_prep_hist(PArgs a) {
         for (int t = 0; t < 4; ++t) pre[t] = sel->pre[t];
     }
     __syncthreads();
-    const int hb = LEVEL == 1 ? st.hb : st.hb2;
-    const int b0 = ((int)blockIdx.x - (LEVEL == 1 ? st.wg_hist : st.wg_hist2)) * hb;
+    const int hb = WD ? st.hb2 : st.hb;
+    const int b0 = ((int)blockIdx.x - (WD ? st.wg_hist2 : st.wg_hist)) * hb;
     const int b1 = min(b0 + hb, st.nblk);
     bool nan = false;
     uint32_t run_bin = 0xffffffffu, run_n = 0u;   // the thread's current run of one histogram index
@@ -628,6 +639,14 @@ __global__ void __launch_bounds__(NT) k_prep_hist(PArgs a) {
             *(float4*)(st.sc + ((int64_t)kk * a.img + dy) * a.img + dx0) = make_float4(v[0], v[1], v[2], v[3]);
         // The UP values of a unit are counted in one step when every counted one continues the
         // thread's run (the common case: no branch taken); otherwise value by value.
+        if constexpr (CP > 1) {
+#pragma unroll
+            for (int i = 0; i < UP; ++i) {
+                nan |= v[i] != v[i];
+                atomicAdd(&s_h[(order_key(v[i]) >> 21) * CP + (threadIdx.x & (CP - 1))], 1u);
+            }
+            return;
+        }
         if constexpr (LEVEL == 1) {
             // a thread's values are neighbours (UP along x, then the next row of its column), so they
             // mostly share a (coarse) level-1 bin: the thread counts a run in a register and adds it
@@ -656,11 +675,15 @@ __global__ void __launch_bounds__(NT) k_prep_hist(PArgs a) {
             return;
         }
         // the keys under one of the slots' prefixes (unused slots hold 0xffffffff, which no key has at
-        // these levels), counted in runs as at level 1 (runs of equal values, e.g. a zero background,
-        // are common); index = slot * NB + bin, slots from NH on count in memory
+        // these levels); index = slot * NB + bin, slots from NH on count in memory.  Keys of the thread's
+        // run (a value four of its neighbours shared, e.g. a zero background) count in a register; any
+        // other adds to LDS by itself and leaves the run: within one level-1 bin the keys spread over the
+        // 2048 finer ones, so lanes seldom meet.  (A run that followed every change of bin broke at
+        // almost every unit of noisy values: level 2 of 8 stacks of 24 x 288^2 26.6 us, with the wide workgroups 21-25; a wave
+        // counting only its uniform units in one add took 88 against 48 us at a study's two levels,
+        // where background and body share waves.)
         uint32_t idx[UP];
-        bool ok[UP], same = true;
-        uint32_t add = 0u;
+        bool ok[UP], one = true;
 #pragma unroll
         for (int i = 0; i < UP; ++i) {
             const uint32_t k = order_key(v[i]);
@@ -669,27 +692,27 @@ __global__ void __launch_bounds__(NT) k_prep_hist(PArgs a) {
             ok[i] = p == pre[0] || p == pre[1] || p == pre[2] || p == pre[3];
             const uint32_t t = p == pre[0] ? 0u : p == pre[1] ? 1u : p == pre[2] ? 2u : 3u;
             idx[i] = t * NB + bin;
-            same &= !ok[i] || idx[i] == run_bin;
-            add += ok[i] ? 1u : 0u;
+            one &= ok[i] && idx[i] == idx[0];
         }
-        if (same) {
-            run_n += add;
-            return;
+        if (one && idx[0] != run_bin) {
+            if (run_n) run_flush();
+            run_bin = idx[0];
+            run_n = 0u;
         }
 #pragma unroll
         for (int i = 0; i < UP; ++i) {
-            if (ok[i]) {
-                if (idx[i] != run_bin) {
-                    if (run_n) run_flush();
-                    run_bin = idx[i];
-                    run_n = 0u;
-                }
-                ++run_n;
+            const bool in = idx[i] == run_bin;
+            run_n += ok[i] && in ? 1u : 0u;
+            if (ok[i] && !in) {
+                if (idx[i] < (uint32_t)(NH * NB))
+                    atomicAdd(&s_h[idx[i]], 1u);
+                else
+                    atomicAdd(gh + idx[i], 1u);
             }
         }
     };
     with_mode<REGION>(st, a, [&](auto m, auto h, auto w) {
-        run_blocks<decltype(m)::value, decltype(h)::value, decltype(w)::value>(st, a, b0, b1, s_st, count);
+        run_blocks<decltype(m)::value, decltype(h)::value, decltype(w)::value, TH>(st, a, b0, b1, s_st, count);
     });
     if (run_n) run_flush();
     if constexpr (LEVEL == 1) {
@@ -697,42 +720,49 @@ __global__ void __launch_bounds__(NT) k_prep_hist(PArgs a) {
     }
     __syncthreads();
     const int nh = LEVEL == 1 ? 1 : min((int)nslot, NH);
-    for (int i = threadIdx.x; i < nh * NB; i += NT) {
-        const uint32_t c = s_h[i];
+    for (int i = threadIdx.x; i < nh * NB; i += TH) {
+        uint32_t c = 0u;
+#pragma unroll
+        for (int k = 0; k < CP; ++k) c += s_h[i * CP + k];
         if (c) atomicAdd(gh + i, c);
     }
 }
 
-// Exclusive prefix sum over the workgroup (one value per thread) and the total.
-DEV uint32_t block_excl_scan(uint32_t x, uint32_t* s_w, uint32_t& total) {
+// Exclusive prefix sums over the workgroup of four values per thread at once.
+DEV void block_excl_scan4(uint32_t (&x)[4], uint32_t (*s_w)[4]) {
     const int lane = __lane_id(), wv = threadIdx.x >> 6;
-    uint32_t incl = x;
+    uint32_t incl[4];
 #pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-        const uint32_t y = __shfl_up(incl, d, 64);
-        if (lane >= d) incl += y;
-    }
-    if (lane == 63) s_w[wv] = incl;
-    __syncthreads();
-    uint32_t base = 0, tot = 0;
+    for (int t = 0; t < 4; ++t) incl[t] = x[t];
 #pragma unroll
-    for (int i = 0; i < NT / 64; ++i) {
-        const uint32_t c = s_w[i];
-        base += i < wv ? c : 0u;
-        tot += c;
-    }
+    for (int d = 1; d < 64; d <<= 1)
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            const uint32_t y = __shfl_up(incl[t], d, 64);
+            if (lane >= d) incl[t] += y;
+        }
+    if (lane == 63)
+#pragma unroll
+        for (int t = 0; t < 4; ++t) s_w[wv][t] = incl[t];
     __syncthreads();
-    total = tot;
-    return base + incl - x;
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+        uint32_t base = 0;
+#pragma unroll
+        for (int i = 0; i < NT / 64; ++i) base += i < wv ? s_w[i][t] : 0u;
+        x[t] = base + incl[t] - x[t];
+    }
 }
 
 // The bins holding the 4 ranks at one level (one workgroup per stack); the last level also derives
-// the percentiles, the scale and the bad flag.
+// the percentiles, the scale and the bad flag.  Latency is its cost (one workgroup, between two passes that
+// wait for it): the four ranks' histograms are loaded together, 16 bytes a load, and scanned together
+// (rank by rank it took 6.1, 6.5 and 4.7 us, now 4.1-4.7 each).
 template <int LEVEL>
 __global__ void __launch_bounds__(NT) k_prep_select(PArgs a) {
     constexpr int NB = LEVEL == 1 ? NB1 : LEVEL == 2 ? NB2 : NB3;
     constexpr int PER = NB / NT;
-    __shared__ uint32_t s_w[NT / 64];
+    __shared__ uint32_t s_w[NT / 64][4];
     __shared__ uint32_t s_bin[4], s_res[4];
     const PStack& st = a.s[blockIdx.x];
     uint32_t rank[4], slot[4] = {0u, 0u, 0u, 0u}, pre[4] = {0u, 0u, 0u, 0u};
@@ -746,22 +776,34 @@ __global__ void __launch_bounds__(NT) k_prep_select(PArgs a) {
     }
     const uint32_t* gh = st.ws + (LEVEL == 1 ? W_H1 : LEVEL == 2 ? W_H2 : W_H3);
     if (threadIdx.x < 4) { s_bin[threadIdx.x] = 0u; s_res[threadIdx.x] = 0u; }
-    for (int t = 0; t < 4; ++t) {
-        const uint32_t* h = gh + slot[t] * NB + threadIdx.x * PER;
-        uint32_t c[PER], sum = 0;
+    static_assert(PER % 4 == 0, "whole 16-byte loads");
+    uint32_t c[4][PER], sum[4], excl[4];
 #pragma unroll
-        for (int i = 0; i < PER; ++i) { c[i] = h[i]; sum += c[i]; }
-        uint32_t total;
-        const uint32_t excl = block_excl_scan(sum, s_w, total);
-        if (excl <= rank[t] && rank[t] < excl + sum) {
-            uint32_t acc = excl;
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int i = 0; i < PER; i += 4) {
+            const uint4 v = *(const uint4*)(gh + slot[t] * NB + threadIdx.x * PER + i);
+            c[t][i] = v.x; c[t][i + 1] = v.y; c[t][i + 2] = v.z; c[t][i + 3] = v.w;
+        }
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+        sum[t] = 0;
+#pragma unroll
+        for (int i = 0; i < PER; ++i) sum[t] += c[t][i];
+        excl[t] = sum[t];
+    }
+    block_excl_scan4(excl, s_w);
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+        if (excl[t] <= rank[t] && rank[t] < excl[t] + sum[t]) {
+            uint32_t acc = excl[t];
 #pragma unroll
             for (int i = 0; i < PER; ++i) {
-                if (rank[t] >= acc && rank[t] < acc + c[i]) {
+                if (rank[t] >= acc && rank[t] < acc + c[t][i]) {
                     s_bin[t] = threadIdx.x * PER + i;
                     s_res[t] = rank[t] - acc;
                 }
-                acc += c[i];
+                acc += c[t][i];
             }
         }
     }
@@ -771,19 +813,27 @@ __global__ void __launch_bounds__(NT) k_prep_select(PArgs a) {
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
         const uint32_t b = s_bin[t];
-        key[t] = LEVEL == 1 ? b : LEVEL == 2 ? ((pre[slot[t]] << 11) | b) : ((pre[slot[t]] << 10) | b);
+        const uint32_t q = slot[t] == 0 ? pre[0] : slot[t] == 1 ? pre[1] : slot[t] == 2 ? pre[2] : pre[3];
+        key[t] = LEVEL == 1 ? b : LEVEL == 2 ? ((q << 11) | b) : ((q << 10) | b);
     }
     if constexpr (LEVEL < 3) {
+        // the distinct keys in order of first use (indexed by constants: no array in memory)
         Sel out;
-        out.nslot = 0;
+        uint32_t nslot = 0;
+#pragma unroll
+        for (int t = 0; t < 4; ++t) out.pre[t] = 0xffffffffu;
+#pragma unroll
         for (int t = 0; t < 4; ++t) {
-            uint32_t j = 0;
-            while (j < out.nslot && out.pre[j] != key[t]) ++j;
-            if (j == out.nslot) out.pre[out.nslot++] = key[t];
+            uint32_t j = nslot;
+#pragma unroll
+            for (int u = t - 1; u >= 0; --u) j = key[u] == key[t] ? out.slot[u] : j;
             out.slot[t] = j;
             out.res[t] = s_res[t];
+#pragma unroll
+            for (int s = 0; s < 4; ++s) out.pre[s] = (uint32_t)s == j ? key[t] : out.pre[s];
+            nslot += j == nslot ? 1u : 0u;
         }
-        for (uint32_t j = out.nslot; j < 4; ++j) out.pre[j] = 0xffffffffu;
+        out.nslot = nslot;
         out.pad_[0] = out.pad_[1] = out.pad_[2] = 0u;
         Sel* dst = (Sel*)(st.ws + (LEVEL == 1 ? W_SEL1 : W_SEL2));
         *dst = out;
@@ -1212,6 +1262,31 @@ PArgs float_view(const PArgs& a) {
     return f;
 }
 
+// The view the wide workgroups read: float32 stacks in blocks of about 16384 pixels (four 16-byte loads a
+// thread of a wide workgroup), as many blocks a workgroup as leave about four workgroups a CU (a study's
+// level 3 takes 38 us so, 44 with two a CU).
+PArgs wide_view(const PArgs& a) {
+    PArgs f = a;
+    const int rb = a.img >= 16384 ? 1 : 16384 / a.img;
+    int64_t blocks = 0;
+    for (int i = 0; i < f.n; ++i) {
+        PStack& p = f.s[i];
+        p.rb = rb;
+        p.bps = (a.img + rb - 1) / rb;
+        p.nblk = (p.k1 - p.k0) * p.bps;
+        blocks += p.nblk;
+    }
+    const int per = (int)std::max<int64_t>(1, blocks / (4 * d8s_host_cu_count()));
+    int wg = 0;
+    for (int i = 0; i < f.n; ++i) {
+        PStack& p = f.s[i];
+        p.hb2 = per;
+        p.wg_hist2 = wg;
+        wg += (p.nblk + per - 1) / per;
+    }
+    return f;
+}
+
 int prepare(const D8sPrepArgs* in, const char* what, bool resize_only, PArgs& a, int& setup_blocks) {
     PREQ(in != nullptr, "null arguments");
     PREQ(in->kind == 0 || in->kind == 1, "kind must be 0 (uint16 regions) or 1 (float32 stacks)");
@@ -1372,29 +1447,19 @@ extern "C" int d8s_prep(const D8sPrepArgs* in, void* stream) {
     hipStream_t st = (hipStream_t)stream;
     const dim3 gs(sb, a.n);
     k_prep_setup<<<gs, NT, 0, st>>>(a, 1);
-    const int gh = grid_of(a, 0), gh2 = grid_of(a, 1), gn = grid_of(a, 2);
-    if (in->kind == 0) {
-        // resize once (with the level-1 count) into the scratch stacks, then the float32 passes
-        k_prep_hist<1, 1, true><<<gh, NT, 0, st>>>(a);
-        k_prep_select<1><<<a.n, NT, 0, st>>>(a);
-        const PArgs f = float_view(a);
-        const int fh2 = grid_of(f, 1), fn = grid_of(f, 2);
-        k_prep_hist<2, 0><<<fh2, NT, 0, st>>>(f);
-        k_prep_select<2><<<f.n, NT, 0, st>>>(f);
-        k_prep_hist<3, 0><<<fh2, NT, 0, st>>>(f);
-        k_prep_select<3><<<f.n, NT, 0, st>>>(f);
-        k_prep_norm<0><<<fn, NT, 0, st>>>(f);
-        (void)gh2;
-        (void)gn;
-    } else {
-        k_prep_hist<1, 0><<<gh, NT, 0, st>>>(a);
-        k_prep_select<1><<<a.n, NT, 0, st>>>(a);
-        k_prep_hist<2, 0><<<gh2, NT, 0, st>>>(a);
-        k_prep_select<2><<<a.n, NT, 0, st>>>(a);
-        k_prep_hist<3, 0><<<gh2, NT, 0, st>>>(a);
-        k_prep_select<3><<<a.n, NT, 0, st>>>(a);
-        k_prep_norm<0><<<gn, NT, 0, st>>>(a);
-    }
+    // kind 0: the resize once (with the level-1 count) into the scratch stacks, then the float32 passes
+    const PArgs f = in->kind == 0 ? float_view(a) : a, w = wide_view(f);
+    const int gw = grid_of(w, 1), gn = grid_of(f, 2);
+    if (in->kind == 0)
+        k_prep_hist<1, 1, true><<<grid_of(a, 0), NT, 0, st>>>(a);
+    else
+        k_prep_hist<1, 0><<<gw, WIDE, 0, st>>>(w);
+    k_prep_select<1><<<a.n, NT, 0, st>>>(a);
+    k_prep_hist<2, 0><<<gw, WIDE, 0, st>>>(w);
+    k_prep_select<2><<<a.n, NT, 0, st>>>(a);
+    k_prep_hist<3, 0><<<gw, WIDE, 0, st>>>(w);
+    k_prep_select<3><<<a.n, NT, 0, st>>>(a);
+    k_prep_norm<0><<<gn, NT, 0, st>>>(f);
     return d8s_host_launched("d8s_prep");
 }
 

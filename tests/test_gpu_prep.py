@@ -189,3 +189,30 @@ def test_payload_missing_series_slots_are_zero(dev):
     for s in range(8):
         assert np.array_equal(got[s], want[s]), (s, int((got[s] != want[s]).sum()))
     assert not got[2].any() and not got[6].any()
+
+
+@pytest.mark.parametrize("r,k,img,kind", [
+    (1, 1, 8, "noise"),              # 64 values: one partial unit batch of a wide workgroup
+    (3, 2, 136, "noise"),            # a last block shorter than the others, three stacks in one grid
+    (2, 5, 256, "background"),       # a large share of zeros beside noise in the same waves
+    (2, 3, 128, "two"),              # two values alternating: every key beside its run
+    (16, 7, 200, "steps"),           # 16 stacks, few distinct values, several in one level-1 bin
+])
+def test_float_levels_counts(dev, r, k, img, kind):
+    """The radix levels of float32 stacks (wide workgroups, the copies of level 1, keys beside a thread's run
+    at levels 2 and 3) at the edges of their blocks and for values that share or miss their bins: the bytes
+    of numpy's percentiles."""
+    print(f"float levels r={r} k={k} img={img} {kind}", flush=True)
+    rng = np.random.default_rng(img + r)
+    x = rng.normal(600, 60, (r, k, img, img)).astype(np.float32)
+    if kind == "background":
+        x = np.where(rng.random(x.shape) < 0.02, x, 0).astype(np.float32)
+        x[:, :, : img // 2] = rng.normal(600, 60, (r, k, img // 2, img)).astype(np.float32)
+    elif kind == "two":
+        x = np.where((np.arange(img) + np.arange(img)[:, None]) % 2 == 0, np.float32(1.5), np.float32(1.5000001))
+        x = np.broadcast_to(x, (r, k, img, img)).astype(np.float32).copy()
+    elif kind == "steps":
+        x = (np.floor(x / 40) * np.float32(0.001)).astype(np.float32)
+    got = hp.to_uint8_hist_batch(torch.from_numpy(x).to(dev)).cpu().numpy()
+    for i in range(r):
+        assert np.array_equal(got[i], P.to_uint8(x[i])), i
