@@ -232,6 +232,11 @@ __global__ void __launch_bounds__(NT) k_head_prod(ProdP p) {
         }
         __syncthreads();
         if (k0 + KC < kend) fetch(k0 + KC);
+        // the chunk's even and odd groups in sums of their own: chains of 32 products, not of the split's
+        // K (the feature dots are the largest term of a logit, and every window rounds by them)
+        f32x4 part[2][2][2];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) part[u >> 2][(u >> 1) & 1][u & 1] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
         for (int g = 0; g < KC / 16; ++g) {
             f32x4 a[2], b[2];
@@ -245,8 +250,12 @@ __global__ void __launch_bounds__(NT) k_head_prod(ProdP p) {
 #pragma unroll
                 for (int t = 0; t < 2; ++t)
 #pragma unroll
-                    for (int c = 0; c < 2; ++c) acc[t][c] = mfma_f32(a[t][i], b[c][i], acc[t][c]);
+                    for (int c = 0; c < 2; ++c) part[g & 1][t][c] = mfma_f32(a[t][i], b[c][i], part[g & 1][t][c]);
         }
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+            for (int c = 0; c < 2; ++c) acc[t][c] += part[0][t][c] + part[1][t][c];
         __syncthreads();
     }
 #pragma unroll
@@ -279,7 +288,8 @@ struct RowsP {
     int M, W, CD, D, S, T, PER, splits;
 };
 
-// the splits' raw sums of NE elements i, i + 64, ..., added in split order, eight splits' loads in flight
+// the splits' raw sums of NE elements i, i + 64, ...: eight splits' loads in flight, their values added in
+// pairs (a fixed order)
 template <int NE>
 DEV void split_sums(float (&x)[NE], const float* src, int64_t stride, int64_t i, int splits) {
 #pragma unroll
@@ -291,9 +301,11 @@ DEV void split_sums(float (&x)[NE], const float* src, int64_t stride, int64_t i,
 #pragma unroll
             for (int e = 0; e < NE; ++e) v[e][u] = src[min(s0 + u, splits - 1) * stride + i + 64 * e];
 #pragma unroll
-        for (int u = 0; u < 8; ++u)
+        for (int e = 0; e < NE; ++e) {
 #pragma unroll
-            for (int e = 0; e < NE; ++e) x[e] += keep(v[e][u], s0 + u < splits);
+            for (int u = 0; u < 8; ++u) v[e][u] = keep(v[e][u], s0 + u < splits);
+            x[e] += ((v[e][0] + v[e][1]) + (v[e][2] + v[e][3])) + ((v[e][4] + v[e][5]) + (v[e][6] + v[e][7]));
+        }
     }
 }
 
