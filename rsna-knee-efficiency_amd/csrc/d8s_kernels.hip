@@ -3749,12 +3749,11 @@ extern "C" int d8s_conv1_pair(const D8sGemmArgs* a, const D8sGemmArgs* b, void* 
 }
 
 template <int TW, int TH, int KSPL, int PT>
-static int conv2_launch(const D8sConv2Args* a, const D8sConv2Args* b, hipStream_t st, int64_t min_tiles) {
+static int conv2_launch(const D8sConv2Args* a, const D8sConv2Args* b, hipStream_t st) {
     using S = C2Shape<TW, TH, KSPL, PT>;
     const int np = b ? 2 : 1;
     const int tiles_x = (a->W + TW - 1) / TW, tiles_y = (a->H + TH - 1) / TH;
     const int64_t total = (int64_t)a->N * tiles_x * tiles_y;            // per problem
-    if (total * np < min_tiles) return -1;
     REQUIRE(total * np < (1ll << 31), "d8s_conv2: too many tiles");
     const int64_t all = total * np < 2 * cu_count() ? total * np : 2 * cu_count();
     int64_t split = (all + np - 1) / np;
@@ -3773,50 +3772,40 @@ static int check_conv2(const D8sConv2Args* a, const char* what) {
 
 // conv2 kernel variants (d8s_conv2_as), the tile shapes TW x TH: 1 32 x 8, 2 32 x 4, 3 32 x 2 (K split
 // in 4), 4 16 x 4, 5 8 x 8, 6 4 x 16, 7 2 x 32, 8 1 x 64 (K split in 4 from 3 on), each taken for maps
-// at least TW wide; 0 the choice below (the widest tile that fits, and for 32-wide tiles the tallest
-// that still gives three tiles per CU).
+// at least TW wide; 0 the choice below (the widest tile that fits, and for 32-wide tiles a height by
+// the number of tiles; a pair's two problems count together).
 static const int C2V_TW[9] = {0, 32, 32, 32, 16, 8, 4, 2, 1};
 
-static int conv2_variant(const D8sConv2Args* a, int variant) {
+static int conv2_variant(const D8sConv2Args* a, int variant, int np = 1) {
     if (variant < 0 || variant > 8) return -1;
     if (variant != 0) return C2V_TW[variant] <= a->W ? variant : -1;
+    // From 32 columns: 32x8 tiles from six per CU (three full rounds of two resident workgroups: 2376
+    // tiles 29.6 us against 32.1 with 32x4's, 2288 27.7 / 30.7, 1536 21.7 / 21.9), 32x4 below, where half
+    // the tile evens out the rounds (880 32x8 tiles 13.4 us, 1584 of 32x4 12.7; 768 17.0, 1536 13.4) and
+    // against 32x2, whose partial sums leave room for one workgroup per CU, the rounds are two to three
+    // times fewer (594 tiles 6.9 us against 13.8, 198 4.5 / 8.1).  At fewer tiles than three quarters of
+    // the CUs both are one round up to 128 (4.3-4.5 / 4.5-4.7 us).
     if (a->W >= 32) {
-        const int64_t enough = 3 * (int64_t)cu_count();
-        if ((int64_t)a->N * ((a->W + 31) / 32) * ((a->H + 7) / 8) >= enough) return 1;
-        if ((int64_t)a->N * ((a->W + 31) / 32) * ((a->H + 3) / 4) >= enough) return 2;
-        return 3;
+        const int64_t cus = cu_count(), col = (int64_t)np * a->N * ((a->W + 31) / 32);
+        if (col * ((a->H + 7) / 8) >= 6 * cus) return 1;
+        return 4 * col * ((a->H + 3) / 4) > 3 * cus ? 2 : 3;
     }
     return a->W >= 16 ? 4 : a->W >= 8 ? 5 : a->W >= 4 ? 6 : a->W >= 2 ? 7 : 8;
 }
 
 static int conv2_dispatch(const D8sConv2Args* a, const D8sConv2Args* b, hipStream_t st, int variant) {
-    if (variant != 0) {
-        REQUIRE(conv2_variant(a, variant) >= 1,
-                "d8s_conv2: variant " + std::to_string(variant) + " is not taken for this shape");
-        switch (variant) {
-            case 1: return conv2_launch<32, 8, 1, 2>(a, b, st, 0);
-            case 2: return conv2_launch<32, 4, 1, 1>(a, b, st, 0);
-            case 3: return conv2_launch<32, 2, 4, 2>(a, b, st, 0);
-            case 4: return conv2_launch<16, 4, 4, 2>(a, b, st, 0);
-            case 5: return conv2_launch<8, 8, 4, 2>(a, b, st, 0);
-            case 6: return conv2_launch<4, 16, 4, 2>(a, b, st, 0);
-            case 7: return conv2_launch<2, 32, 4, 2>(a, b, st, 0);
-            default: return conv2_launch<1, 64, 4, 2>(a, b, st, 0);
-        }
+    const int v = conv2_variant(a, variant, b ? 2 : 1);
+    REQUIRE(v >= 1, "d8s_conv2: variant " + std::to_string(variant) + " is not taken for this shape");
+    switch (v) {
+        case 1: return conv2_launch<32, 8, 1, 2>(a, b, st);
+        case 2: return conv2_launch<32, 4, 1, 1>(a, b, st);
+        case 3: return conv2_launch<32, 2, 4, 2>(a, b, st);
+        case 4: return conv2_launch<16, 4, 4, 2>(a, b, st);
+        case 5: return conv2_launch<8, 8, 4, 2>(a, b, st);
+        case 6: return conv2_launch<4, 16, 4, 2>(a, b, st);
+        case 7: return conv2_launch<2, 32, 4, 2>(a, b, st);
+        default: return conv2_launch<1, 64, 4, 2>(a, b, st);
     }
-    const int64_t enough = 3 * (int64_t)cu_count();        // tiles for a persistent grid to pipeline
-    if (a->W >= 32) {
-        int rc = conv2_launch<32, 8, 1, 2>(a, b, st, enough);
-        if (rc >= 0) return rc;
-        rc = conv2_launch<32, 4, 1, 1>(a, b, st, enough);
-        if (rc >= 0) return rc;
-        return conv2_launch<32, 2, 4, 2>(a, b, st, 0);
-    }
-    if (a->W >= 16) return conv2_launch<16, 4, 4, 2>(a, b, st, 0);
-    if (a->W >= 8) return conv2_launch<8, 8, 4, 2>(a, b, st, 0);
-    if (a->W >= 4) return conv2_launch<4, 16, 4, 2>(a, b, st, 0);
-    if (a->W >= 2) return conv2_launch<2, 32, 4, 2>(a, b, st, 0);
-    return conv2_launch<1, 64, 4, 2>(a, b, st, 0);
 }
 
 extern "C" int d8s_conv2(const D8sConv2Args* a, void* stream) {

@@ -312,3 +312,12 @@ def test_kernel_variant_queries():
     assert "variant 1" in lib.d8s_last_error().decode()
     assert lib.d8s_transition_as(trans(24, 1024, 32, 8, 38, 640), 1, None) == 1
     assert lib.d8s_conv1_as(big, 2, None) == 1
+
+
+@pytest.mark.parametrize("n,h,w,variant", [(128, 32, 96, 1), (127, 32, 96, 2), (49, 16, 32, 2), (48, 16, 32, 3),
+                                           (11, 36, 36, 2), (1, 1, 32, 3), (5, 7, 31, 4)])
+def test_conv2_choice_by_tiles(n, h, w, variant):
+    """256 CUs: 32x8 tiles from 1536 of them, 32x4 while more than 192, 32x2 below, 16x4 under 32 columns."""
+    lib = hip.library()
+    a = hip.Conv2Args(0x1000, 0x1000, 0x1000, 0x1000, 0x1000, n, h, w, 0)
+    assert lib.d8s_conv2_variant(ctypes.byref(a), 0) == variant
