@@ -102,7 +102,7 @@ def agree(a: np.ndarray, b: np.ndarray) -> dict:
 def kernel_bytes(meta: dict, n: int, kinds: dict | None = None) -> dict[str, list[float]]:
     """Algorithmic HBM bytes of every launch of a pass of n images, per kernel family: compulsory reads
     of the activations and writes of the outputs, plus the weights and tables (read once).  `kinds`
-    {block: "conv" | "chain" | "tile" | "img" | "parts"} (`Dense8SEncoder.fused`): a fused layer
+    {block: "conv" | "chain" | "tile" | "img" | "parts" | "bands"} (`Dense8SEncoder.fused`): a fused layer
     ("dense") has no bottleneck in memory; a chained launch ("chain": conv2 of a layer and conv1 of the
     next) does not read the new layer's channels back; a whole block ("block") reads its input and
     writes its layers' outputs once."""
@@ -136,7 +136,7 @@ def kernel_bytes(meta: dict, n: int, kinds: dict | None = None) -> dict[str, lis
                     out["chain"].append(M * 128 + M * 32 + 36864 + 32 * 8 + c1 - M * 32)
                 if li == b["L"] - 1:
                     out["conv2"].append(c2)
-        if kind in ("img", "parts"):
+        if kind in ("img", "parts", "bands"):
             out["block"].append(M * b["c0"] + M * 32 * b["L"] + wts)
         ctot = b["c0"] + 32 * b["L"]
         if b["trans"]:
@@ -732,7 +732,7 @@ def c4_roofline(enc, reps: int, peak_tops: float | None) -> dict:
         bi = int(label[5:])
         byts, ops = block_work(enc.meta["blocks"][bi], enc.nb)
         tops = ops / (ms * 1e-3) / 1e12
-        out.update({"entry": "d8s_dense_block_parts" if enc.fused[bi].startswith("parts") else "d8s_dense_block",
+        out.update({"entry": "d8s_dense_block_" + enc.fused[bi].split(":")[0] if ":" in enc.fused[bi] else "d8s_dense_block",
                     "kind": enc.fused[bi], "bound": "mfma", "achieved": round(tops, 1), "peak": I8_PEAK_TOPS,
                     "unit": "TOP/s", "frac": round(tops / I8_PEAK_TOPS, 4),
                     "gbs": round(byts / (ms * 1e-3) / 1e9, 1), "algorithmic_bytes": int(byts), "ops": ops})
