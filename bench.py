@@ -914,10 +914,11 @@ FP32_PEAK_TFLOPS = 157.3     # MI355X fp32, published
 
 
 def head_flops(w: int, d: int = 1664, cd: int = 256, ff: int = 512, t: int = 12) -> float:
-    """Multiply-adds x 2 of the head for one study of w windows (ctx_in, in_proj, attention, out_proj,
-    feed-forward, ctx_out, the attention and classifier dots)."""
-    mac = w * d * cd + w * cd * 3 * cd + 2 * w * w * cd + w * cd * cd + 2 * w * cd * ff + w * cd * d \
-        + 2 * w * d * t
+    """Multiply-adds x 2 that d8s_head makes for one study of w windows (ctx_in and the feature dots,
+    in_proj, attention, out_proj, ff1, the dots' weights folded through ctx_out and ff2 and the dots with
+    them; Mo and Mf are made once per call, counted per study here)."""
+    mac = w * d * (cd + 2 * t) + w * cd * 3 * cd + 2 * w * w * cd + w * cd * cd + w * cd * ff \
+        + 2 * t * w * (cd + ff) + 2 * t * cd * (d + ff)
     return 2.0 * mac
 
 
