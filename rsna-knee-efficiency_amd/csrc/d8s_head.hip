@@ -26,7 +26,7 @@
 //
 // The products run on v_mfma_f32_16x16x4_f32 with 16-byte operand reads: lane l holds row (A) or column (B)
 // l % 16 and, in step s of a 16-deep group, k = 4 (l / 16) + s, the same permutation of k for both.
-// Measured with HIP events per call (every input resident): 8 studies of 88 windows 63 us,
+// Measured with HIP events per call (every input resident): 8 studies of 88 windows 65 us,
 // 1 study of 44 windows 49 us (15 launches with the products staged through LDS: 118 and 79 us).
 #include <hip/hip_runtime.h>
 
