@@ -1103,7 +1103,7 @@ template <int KIND>
 constexpr int G4IMG = KIND == 1 ? 4 : 8;     // images per thread
 
 template <int KIND>
-__global__ void __launch_bounds__(NT) k_grid_sample4(D8sGridArgs a) {
+__global__ void __launch_bounds__(NT) k_grid_sample4(D8sGridArgs a, int n_first) {
     constexpr int NI = G4IMG<KIND>;
     __shared__ __attribute__((aligned(16))) float s_lut[KIND == 1 ? 256 * NC : 4];
     if constexpr (KIND == 1) {
@@ -1114,8 +1114,9 @@ __global__ void __launch_bounds__(NT) k_grid_sample4(D8sGridArgs a) {
     }
     const int HW = a.H * a.W;
     const int per = (int)gridDim.x / 8;                       // (gridDim.x is a multiple of 8)
+    // (at most 2^31 - 4: H * W < 2^31 makes at most 2^21 blocks, itself a multiple of 8)
     const int p0 = 4 * ((((int)blockIdx.x % 8) * per + (int)blockIdx.x / 8) * NT + (int)threadIdx.x);
-    const int n0 = blockIdx.y * NI, n1 = min(n0 + NI, a.N);
+    const int n0 = n_first + (int)blockIdx.y * NI, n1 = min(n0 + NI, a.N);
     if (p0 >= HW) return;
     int64_t pl[NI];
 #pragma unroll
@@ -1495,10 +1496,15 @@ extern "C" int d8s_grid_sample(const D8sGridArgs* a, void* stream) {
         // four pixels a thread: rows of whole dwords (uint8 and fp16 alike), the grid's and output's quads
         // aligned
         const unsigned gx = (unsigned)((HW / 4 + NT - 1) / NT + 7) / 8 * 8;
-        if (a->kind == 1)
-            k_grid_sample4<1><<<dim3(gx, (unsigned)((a->N + G4IMG<1> - 1) / G4IMG<1>)), NT, 0, st>>>(*a);
-        else
-            k_grid_sample4<0><<<dim3(gx, (unsigned)((a->N + G4IMG<0> - 1) / G4IMG<0>)), NT, 0, st>>>(*a);
+        // (a grid has at most 65535 y blocks: more images take further launches)
+        const int ni = a->kind == 1 ? G4IMG<1> : G4IMG<0>;
+        for (int n0 = 0; n0 < a->N; n0 += 65535 * ni) {
+            const dim3 g4(gx, (unsigned)std::min(65535, (a->N - n0 + ni - 1) / ni));
+            if (a->kind == 1)
+                k_grid_sample4<1><<<g4, NT, 0, st>>>(*a, n0);
+            else
+                k_grid_sample4<0><<<g4, NT, 0, st>>>(*a, n0);
+        }
     } else if (a->kind == 1) {
         k_grid_sample<1><<<grid, NT, 0, st>>>(*a);
     } else {
