@@ -971,13 +971,15 @@ DEV Tap grid_tap(const D8sGridArgs& a, uint32_t gbits) {
     const float iy = __builtin_fmaf(gy + 1.0f, (float)a.H, -1.0f) * 0.5f;
     t.x0 = (int)floorf(ix);
     t.y0 = (int)floorf(iy);
-    const int x1 = t.x0 + 1, y1 = t.y0 + 1;
+    // (an infinite coordinate saturates: + 1 and the range checks are unsigned, so it wraps to outside.  Signed,
+    // the compiler takes x1 >= 0 as x0 > -2, and the tap at INT_MAX + 1 counted as inside)
+    const int x1 = (int)((uint32_t)t.x0 + 1u), y1 = (int)((uint32_t)t.y0 + 1u);
     t.w[0] = ((float)x1 - ix) * ((float)y1 - iy);
     t.w[1] = (ix - (float)t.x0) * ((float)y1 - iy);
     t.w[2] = ((float)x1 - ix) * (iy - (float)t.y0);
     t.w[3] = (ix - (float)t.x0) * (iy - (float)t.y0);
-    const bool vx0 = t.x0 >= 0 && t.x0 < a.W, vx1 = x1 >= 0 && x1 < a.W;
-    const bool vy0 = t.y0 >= 0 && t.y0 < a.H, vy1 = y1 >= 0 && y1 < a.H;
+    const bool vx0 = (uint32_t)t.x0 < (uint32_t)a.W, vx1 = (uint32_t)x1 < (uint32_t)a.W;
+    const bool vy0 = (uint32_t)t.y0 < (uint32_t)a.H, vy1 = (uint32_t)y1 < (uint32_t)a.H;
     t.ok[0] = vy0 && vx0;
     t.ok[1] = vy0 && vx1;
     t.ok[2] = vy1 && vx0;
@@ -1134,9 +1136,9 @@ __global__ void __launch_bounds__(NT) k_grid_sample4(D8sGridArgs a, int n_first)
     bool in = rows, out = rows;
 #pragma unroll
     for (int k = 1; k < 4; ++k) {
-        const int o = t[k].x0 - x0;
-        in &= o == k - 1 || o == k;
-        out &= o == k || o == k + 1;
+        const uint32_t o = (uint32_t)t[k].x0 - (uint32_t)x0;   // (x0 may lie anywhere)
+        in &= o == (uint32_t)k - 1 || o == (uint32_t)k;
+        out &= o == (uint32_t)k || o == (uint32_t)k + 1;
     }
     // (a zoom out's columns x0 .. x0 + 5 may reach into a third dword of bytes)
     out &= KIND == 0 || base <= a.W - 12;

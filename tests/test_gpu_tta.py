@@ -191,3 +191,36 @@ def test_grid_sample_many_images(dev, kind):
     want = torch.cat([F.grid_sample(c[:, None], grid.expand(len(c), h, w, 2), mode="bilinear", padding_mode="zeros",
                                     align_corners=False)[:, 0] for c in imgs.split(65536)])
     assert torch.equal(out, want[idx] if kind == 1 else want)
+
+
+@pytest.mark.parametrize("kind", [0, 1])
+@pytest.mark.parametrize("h,w", [(9, 12), (40, 256), (21, 61)])
+def test_grid_sample_infinite_coordinates(dev, kind, h, w):
+    """Infinite coordinates beside ordinary ones (a scale past fp16's range): those pixels have no tap inside
+    the image and are zero, the others are torch's grid_sample."""
+    import ctypes
+    from rsna_knee_efficiency_amd import hip
+    n, sk = 11, 5
+    print(f"infinite coordinates kind={kind} {h}x{w}", flush=True)
+    g = torch.Generator().manual_seed(h * w)
+    grid = tta.view_grid(h, w, 1, 1.1, 0.0, 0.0, torch.float16, dev).clone()
+    bad = (torch.rand((h, w, 2), generator=g) < 0.05).to(dev)
+    ordinary = grid.clone()
+    grid[bad] = float("inf")
+    grid[1::2][bad[1::2]] = float("-inf")
+    lut = tta.lut_u8_f16(dev)
+    idx = torch.randint(0, sk, (n,), generator=g).to(dev)
+    if kind == 1:
+        src = torch.randint(0, 256, (sk, h, w), generator=g, dtype=torch.uint8).to(dev)
+        imgs = lut[src[idx].long()]
+    else:
+        src = torch.rand((n, h, w), generator=g).half().to(dev)
+        imgs = src
+    want = F.grid_sample(imgs[:, None], ordinary.expand(n, h, w, 2), mode="bilinear", padding_mode="zeros",
+                         align_corners=False)[:, 0]
+    want[:, bad.any(2)] = 0
+    out = torch.full((n, h, w), 9.0, dtype=torch.float16, device=dev)
+    a = hip.GridArgs(src=src.data_ptr(), slice_idx=idx.data_ptr(), lut=lut.data_ptr(), grid=grid.data_ptr(),
+                     out=out.data_ptr(), kind=kind, N=n, H=h, W=w, B=1, SK=sk, M=n)
+    hip.call("d8s_grid_sample", ctypes.byref(a), ctypes.c_void_p(torch.cuda.current_stream(dev).cuda_stream))
+    assert torch.equal(out, want)
