@@ -956,6 +956,13 @@ DEV void nt_store64(void* p, uint32_t lo, uint32_t hi) {
     __builtin_nontemporal_store((uint64_t)lo | (uint64_t)hi << 32, (uint64_t*)p);
 }
 
+// The fp16 bits of a float32 sum, which is opaque here: a conversion that the compiler sees behind an fma becomes
+// one v_fma_mixlo_f16, which rounds once where the sum is to be rounded to float32 first.
+DEV uint32_t half_bits(float x) {
+    asm("" : "+v"(x));
+    return (uint32_t)__half_as_ushort(__float2half_rn(x));
+}
+
 // Taps (nw, ne, sw, se), weights and which taps lie inside the image, of one output pixel.
 struct Tap {
     int x0, y0;
@@ -1031,7 +1038,7 @@ __global__ void __launch_bounds__(NT) k_grid_sample(D8sGridArgs a) {
     grid_pixel<KIND, GIMG>(a, t, pl, acc, [&](uint32_t u) { return __half2float(__ushort_as_half(s_lut[u])); });
 #pragma unroll
     for (int i = 0; i < GIMG; ++i)
-        if (n0 + i < n1) ((__half*)a.out)[(int64_t)(n0 + i) * HW + p] = __float2half_rn(acc[i]);
+        if (n0 + i < n1) ((uint16_t*)a.out)[(int64_t)(n0 + i) * HW + p] = (uint16_t)half_bits(acc[i]);
 }
 
 // The gather alone (no grid): out = lut[slice], 8 consecutive pixels of a plane per thread (the last of a
@@ -1089,23 +1096,36 @@ __global__ void __launch_bounds__(NT) k_grid_gather(D8sGridArgs a) {
 }
 
 // Four consecutive output pixels of a row per thread (W a multiple of 4, the grid 16-byte aligned).  Where
-// the four share their two source rows inside the image and their left taps advance by at most one column
-// a pixel (a zoom in, a shift: o_k in {k - 1, k} from the first's), or by at least one (a zoom out of less
-// than a third: {k, k + 1}), their taps are at most 5 (6) columns of the two rows: two dwords (KIND 0: 16
-// bytes) per row and image, each column converted once, a pixel's two picked by one select a row.
-// Elsewhere each pixel takes the one-pixel kernel's taps.  Per pixel the values, weights and fma order are
-// the one-pixel kernel's, so the outputs are identical.  What bounded the uint8 form was the table in LDS:
-// sixteen lookups of random entries a thread and image, about four lanes on one bank each; now ten (twelve)
-// in a table of NC float32 copies, a lane's
-// copy by its index, and streaming stores (88 x 3 windows of 512 x 512: 101 -> 82 us, zoomed out 180 -> 148;
-// fp16 images, which had one pixel a thread, 92 -> 50).  The grid's x blocks are renumbered so
-// that each XCD's share is consecutive rows (neighbouring blocks read the same source rows: one L2).
+// the four share their two source rows inside the image, their taps lie in a few columns of the two rows from
+// the least left column on: two or three dwords (KIND 0: four or five) per row and image, each column converted
+// once, a pixel's two picked by selects.  By o_k, pixel k's left column from the least:
+//   NEAR  o_k in {k - 1, k}: zooms in up to about 1.6, shifts; 5 columns, a select a row and pixel;
+//   IN    any o_k up to 3: further zooms in, mirrored images; 5 columns, three selects;
+//   OUT   o_k in {k, k + 1}: zooms out to about 0.75; 6 columns, one select;
+//   FAR   o_k in k .. 2 k: zooms out to 0.5; 8 columns, k selects.
+// Pixels whose taps all lie outside the image store zeros; the others (borders, further zooms out, rotations)
+// take the one-pixel kernel's taps, for fp16 images a lane per pixel where more than 8 lanes of a wave need it.
+// A wave all NEAR decides nothing else; the lanes of any other take one form together where one fits.
+// Per pixel the values, weights and fma order are the one-pixel kernel's, so the outputs are identical.
+// What bounds the uint8 form is the table in LDS: ten to sixteen lookups of random entries a thread and image
+// (sixteen through one table: about four lanes on one bank each), in a table of NC float32 copies, a lane's
+// copy by its index; streaming stores leave the caches to the source.  88 x 3 windows, us by scale, this
+// kernel and (in brackets) a single window rule of 8 aligned bytes for uint8, a pixel a thread for fp16:
+//   uint8 512 px  0.5 92 (82)  0.7 109 (156)  0.9 108 (143)  1.1 52 (61)  1.8 65 (60)  2.5 65 (59)  -1.1 67 (60)
+//   uint8 288 px  0.5 42 (34)  0.7 43 (66)    0.9 41 (55)    1.1 20 (27)  1.8 26 (27)  2.5 26 (27)  -1.1 27 (27)
+//   fp16  288 px  0.4 35 (26)  0.5 31 (29)  0.7 38 (36)  0.9 29 (42)  1.1 16 (29)  2.5 19 (25)  -1.1 21 (29)
+// The grid's x blocks are renumbered so that each XCD's share is consecutive rows (neighbouring blocks read the
+// same source rows: one L2).
 constexpr int NC = 16;
 template <int KIND>
 constexpr int G4IMG = KIND == 1 ? 4 : 8;     // images per thread
+enum { NEAR, OUT, IN, FAR };
+// pixel k's least left column, and how many further ones it may take
+constexpr int lo_of(int mode, int k) { return mode == NEAR ? (k ? k - 1 : 0) : mode == IN ? 0 : k; }
+constexpr int steps_of(int mode, int k) { return mode == IN ? 3 : mode == FAR ? k : k ? 1 : 0; }
 
 template <int KIND>
-__global__ void __launch_bounds__(NT) k_grid_sample4(D8sGridArgs a, int n_first) {
+__global__ void __launch_bounds__(NT, KIND == 1 ? 7 : 4) k_grid_sample4(D8sGridArgs a, int n_first) {
     constexpr int NI = G4IMG<KIND>;
     __shared__ __attribute__((aligned(16))) float s_lut[KIND == 1 ? 256 * NC : 4];
     if constexpr (KIND == 1) {
@@ -1129,83 +1149,149 @@ __global__ void __launch_bounds__(NT) k_grid_sample4(D8sGridArgs a, int n_first)
     auto lut = [&](uint32_t at) {                             // at = 4 NC u
         return *(const float*)((const char*)s_lut + (at | lane_off));
     };
-    const int x0 = t[0].x0, y0 = t[0].y0;
+    const int y0 = t[0].y0, x0 = t[0].x0;
     constexpr int AL = KIND == 1 ? 4 : 2;                     // pixels per dword
-    const int base = x0 & ~(AL - 1);
-    const bool rows = t[1].y0 == y0 && t[2].y0 == y0 && t[3].y0 == y0 && y0 >= 0 && y0 < a.H - 1 && x0 >= 0 && base <= a.W - 8;
-    bool in = rows, out = rows;
+    const bool same = t[1].y0 == y0 && t[2].y0 == y0 && t[3].y0 == y0 && y0 >= 0 && y0 < a.H - 1;
+    // what a lane's taps allow: near (here), in / out / far / none (further down)
+    bool near = same && x0 >= 0 && (x0 & ~(AL - 1)) <= a.W - 8;
 #pragma unroll
-    for (int k = 1; k < 4; ++k) {
-        const uint32_t o = (uint32_t)t[k].x0 - (uint32_t)x0;   // (x0 may lie anywhere)
-        in &= o == (uint32_t)k - 1 || o == (uint32_t)k;
-        out &= o == (uint32_t)k || o == (uint32_t)k + 1;
-    }
-    // (a zoom out's columns x0 .. x0 + 5 may reach into a third dword of bytes)
-    out &= KIND == 0 || base <= a.W - 12;
+    for (int k = 1; k < 4; ++k) near &= (uint32_t)k - ((uint32_t)t[k].x0 - (uint32_t)x0) <= 1u;
     float acc[NI][4];
-    // SH: pixel k's left column is k - 1 + SH or k + SH
-    auto fast = [&](auto sh) __attribute__((always_inline)) {
-        constexpr int SH = decltype(sh)::value, COLS = 5 + SH;
-        const int r0 = y0 * a.W + base;
-        constexpr int DW = KIND == 1 ? 2 + SH : 4;
-        uint32_t d[NI][2][DW];
+    // x: the least of the four left columns
+    auto fast = [&](auto mode, int x) __attribute__((always_inline)) {
+        constexpr int MODE = decltype(mode)::value, COLS = MODE == FAR ? 8 : MODE == OUT ? 6 : 5;
+        constexpr int DW = KIND == 0 ? (COLS + 3) / 2 : COLS == 5 ? 2 : 3;
+        constexpr int CI = KIND == 0 && MODE == FAR ? NI / 2 : NI;   // images whose dwords are in registers together
+        const int r0 = y0 * a.W + (x & ~(AL - 1));
+        const uint32_t sft = (uint32_t)(x & (AL - 1)) * (KIND == 1 ? 8 : 16);
+        // pixel k's left column is LO + (how many of is[k][] hold)
+        constexpr int STEPS = MODE == IN || MODE == FAR ? 3 : 1;
+        bool is[4][STEPS];
 #pragma unroll
-        for (int i = 0; i < NI; ++i)
+        for (int k = 0; k < 4; ++k)
 #pragma unroll
-            for (int r = 0; r < 2; ++r) {
-                const uint32_t* q = (const uint32_t*)((const uint8_t*)a.src + (KIND == 1 ? 1 : 2) * (pl[i] + r0 + r * a.W));
+            for (int e = 0; e < STEPS; ++e) is[k][e] = t[k].x0 - x > lo_of(MODE, k) + e;
 #pragma unroll
-                for (int w = 0; w < DW; ++w) d[i][r][w] = q[w];
-            }
-        const uint32_t sft = (uint32_t)(x0 - base) * (KIND == 1 ? 8 : 16);
-        bool up[4];
+        for (int i0 = 0; i0 < NI; i0 += CI) {
+            uint32_t d[CI][2][DW];
 #pragma unroll
-        for (int k = 0; k < 4; ++k) up[k] = t[k].x0 - x0 == k + SH;
-#pragma unroll
-        for (int i = 0; i < NI; ++i) {
-            float c[2][COLS + (COLS & 1)];
-#pragma unroll
-            for (int r = 0; r < 2; ++r) {
-                if constexpr (KIND == 1) {
-                    const uint32_t lo = __builtin_amdgcn_alignbit(d[i][r][1], d[i][r][0], sft);
-                    const uint32_t hi = __builtin_amdgcn_alignbit(d[i][r][DW - 1], d[i][r][1], sft);
-                    constexpr uint32_t M = 255u * 4 * NC;
-                    static_assert(NC == 16, "byte u at bit 6: 4 NC u");
-                    c[r][0] = lut((lo << 6) & M);
-                    c[r][1] = lut((lo >> 2) & M);
-                    c[r][2] = lut((lo >> 10) & M);
-                    c[r][3] = lut((lo >> 18) & M);
-                    c[r][4] = lut((hi << 6) & M);
-                    if constexpr (COLS > 5) c[r][5] = lut((hi >> 2) & M);
-                } else {
-#pragma unroll
-                    for (int w = 0; w < 3; ++w) {
-                        const __half2 v = __builtin_bit_cast(__half2, __builtin_amdgcn_alignbit(d[i][r][w + 1], d[i][r][w], sft));
-                        c[r][2 * w] = __low2float(v);
-                        if (2 * w + 1 < COLS) c[r][2 * w + 1] = __high2float(v);
-                    }
-                }
-            }
-#pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                float s = 0.0f;
+            for (int i = 0; i < CI; ++i)
 #pragma unroll
                 for (int r = 0; r < 2; ++r) {
-                    // (pixel 0 of a zoom in has o = 0: column 0; of a zoom out 0 too)
-                    const int lo = k - 1 + SH;
-                    const float l = lo < 0 || (SH == 1 && k == 0) ? c[r][0] : up[k] ? c[r][lo + 1] : c[r][lo];
-                    const float h = lo < 0 || (SH == 1 && k == 0) ? c[r][1] : up[k] ? c[r][lo + 2] : c[r][lo + 1];
-                    s = __builtin_fmaf(l, t[k].w[2 * r], s);
-                    s = __builtin_fmaf(h, t[k].w[2 * r + 1], s);
+                    const uint32_t* q = (const uint32_t*)((const uint8_t*)a.src + (KIND == 1 ? 1 : 2) * (pl[i0 + i] + r0 + r * a.W));
+#pragma unroll
+                    for (int w = 0; w < DW; ++w) d[i][r][w] = q[w];
                 }
-                acc[i][k] = s;
+#pragma unroll
+            for (int i = 0; i < CI; ++i) {
+                float c[2][COLS + (COLS & 1)];
+#pragma unroll
+                for (int r = 0; r < 2; ++r) {
+                    if constexpr (KIND == 1) {
+                        const uint32_t lo = __builtin_amdgcn_alignbit(d[i][r][1], d[i][r][0], sft);
+                        const uint32_t hi = __builtin_amdgcn_alignbit(d[i][r][DW - 1], d[i][r][1], sft);
+                        constexpr uint32_t M = 255u * 4 * NC;
+                        static_assert(NC == 16, "byte u at bit 6: 4 NC u");
+                        c[r][0] = lut((lo << 6) & M);
+                        c[r][1] = lut((lo >> 2) & M);
+                        c[r][2] = lut((lo >> 10) & M);
+                        c[r][3] = lut((lo >> 18) & M);
+                        c[r][4] = lut((hi << 6) & M);
+                        if constexpr (COLS > 5) c[r][5] = lut((hi >> 2) & M);
+                        if constexpr (COLS > 6) c[r][6] = lut((hi >> 10) & M);
+                        if constexpr (COLS > 6) c[r][7] = lut((hi >> 18) & M);
+                    } else {
+#pragma unroll
+                        for (int w = 0; w < DW - 1; ++w) {
+                            const __half2 v = __builtin_bit_cast(__half2, __builtin_amdgcn_alignbit(d[i][r][w + 1], d[i][r][w], sft));
+                            c[r][2 * w] = __low2float(v);
+                            if (2 * w + 1 < COLS) c[r][2 * w + 1] = __high2float(v);
+                        }
+                    }
+                }
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    float s = 0.0f;
+#pragma unroll
+                    for (int r = 0; r < 2; ++r) {
+                        const int lo = lo_of(MODE, k);
+                        float l = c[r][lo], h = c[r][lo + 1];
+#pragma unroll
+                        for (int e = 0; e < steps_of(MODE, k); ++e) {
+                            l = is[k][e] ? c[r][lo + e + 1] : l;
+                            h = is[k][e] ? c[r][lo + e + 2] : h;
+                        }
+                        s = __builtin_fmaf(l, t[k].w[2 * r], s);
+                        s = __builtin_fmaf(h, t[k].w[2 * r + 1], s);
+                    }
+                    acc[i0 + i][k] = s;
+                }
             }
         }
     };
-    if (in) {
-        fast(std::integral_constant<int, 0>{});
-    } else if (out) {
-        fast(std::integral_constant<int, 1>{});
+    // (an image past the last is the last again: a store under a branch would take its loads there with it)
+    auto store = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < NI; ++i) {
+            const uint32_t lo = half_bits(acc[i][0]) | half_bits(acc[i][1]) << 16;
+            const uint32_t hi = half_bits(acc[i][2]) | half_bits(acc[i][3]) << 16;
+            nt_store64((uint16_t*)a.out + (int64_t)min(n0 + i, n1 - 1) * HW + p0, lo, hi);
+        }
+    };
+    if (__all(near)) {
+        fast(std::integral_constant<int, NEAR>{}, x0);
+        store();
+        return;
+    }
+    const int xmin = min(min(x0, t[1].x0), min(t[2].x0, t[3].x0)), xmax = max(max(x0, t[1].x0), max(t[2].x0, t[3].x0));
+    const int base = xmin & ~(AL - 1);
+    const bool rows = same && xmin >= 0 && base <= a.W - 8;
+    bool in = rows && (uint32_t)xmax - (uint32_t)xmin <= 3u, out = rows, far = rows, none = true;
+    {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const uint32_t o = (uint32_t)t[k].x0 - (uint32_t)xmin;
+            out &= o == (uint32_t)k || (k > 0 && o == (uint32_t)k + 1u);
+            far &= o >= (uint32_t)k && o <= 2u * k;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) none &= !t[k].ok[q];
+        }
+        // (a zoom out's columns may reach into a further dword)
+        out &= KIND == 0 || base <= a.W - 12;
+        far &= base <= a.W - (KIND == 1 ? 12 : 10);
+        if constexpr (KIND == 0) {
+            const bool slow = !(in || out || far || none);
+            if (__popcll(__ballot(slow)) > 8 && __ballot(true) == ~0ull) {
+                // much of the wave has taps that lie nowhere together: a lane per pixel, 64 neighbours at a time
+                const int pw = p0 - 3 * (int)__lane_id();
+#pragma unroll 2
+                for (int s = 0; s < 256; s += 64) {
+                    const Tap ts = grid_tap(a, ((const uint32_t*)a.grid)[pw + s]);
+                    float v[NI];
+                    grid_pixel<KIND, NI>(a, ts, pl, v, lut);
+#pragma unroll
+                    for (int i = 0; i < NI; ++i)
+                        ((uint16_t*)a.out)[(int64_t)min(n0 + i, n1 - 1) * HW + pw + s] = (uint16_t)half_bits(v[i]);
+                }
+                return;
+            }
+        }
+        // one form for the wave's lanes where one will do (a lane's neighbours often need the wider form)
+    }
+    const bool use_in = __any(in && !near && !out), use_out = __any(out && !near), use_far = __any(far && !out && !in);
+    if (use_far && far) {
+        fast(std::integral_constant<int, FAR>{}, xmin);
+    } else if (use_out && out) {
+        fast(std::integral_constant<int, OUT>{}, xmin);
+    } else if (use_in && in) {
+        fast(std::integral_constant<int, IN>{}, xmin);
+    } else if (near) {
+        fast(std::integral_constant<int, NEAR>{}, x0);
+    } else if (none) {
+#pragma unroll
+        for (int i = 0; i < NI; ++i)
+#pragma unroll
+            for (int k = 0; k < 4; ++k) acc[i][k] = 0.0f;
     } else {
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
@@ -1215,15 +1301,7 @@ __global__ void __launch_bounds__(NT) k_grid_sample4(D8sGridArgs a, int n_first)
             for (int i = 0; i < NI; ++i) acc[i][k] = v[i];
         }
     }
-#pragma unroll
-    for (int i = 0; i < NI; ++i)
-        if (n0 + i < n1) {
-            const uint32_t lo = (uint32_t)__half_as_ushort(__float2half_rn(acc[i][0])) |
-                                ((uint32_t)__half_as_ushort(__float2half_rn(acc[i][1])) << 16);
-            const uint32_t hi = (uint32_t)__half_as_ushort(__float2half_rn(acc[i][2])) |
-                                ((uint32_t)__half_as_ushort(__float2half_rn(acc[i][3])) << 16);
-            nt_store64((uint16_t*)a.out + (int64_t)(n0 + i) * HW + p0, lo, hi);
-        }
+    store();
 }
 
 // ---- host side ----------------------------------------------------------------------------------

@@ -224,3 +224,51 @@ def test_grid_sample_infinite_coordinates(dev, kind, h, w):
                      out=out.data_ptr(), kind=kind, N=n, H=h, W=w, B=1, SK=sk, M=n)
     hip.call("d8s_grid_sample", ctypes.byref(a), ctypes.c_void_p(torch.cuda.current_stream(dev).cuda_stream))
     assert torch.equal(out, want)
+
+
+@pytest.mark.parametrize("kind", [0, 1])
+@pytest.mark.parametrize("h,w", [(9, 12), (40, 256), (37, 60)])
+@pytest.mark.parametrize("view", [1.8, 2.5, 4.0, 0.75, 0.55, 0.5, 0.4, 0.25, -1.0, -1.3, -0.6, "turn", "noise", "nan"])
+def test_grid_sample_forms(dev, kind, h, w, view):
+    """Every form of the four-pixel kernel: zooms in and out of any scale, mirrored images, a rotation, a grid of
+    noise (no taps together) and one with NaN and infinite coordinates beside ordinary ones, where a wave's
+    lanes differ; a group remainder of images.  Bit for bit the one-pixel form, and torch's grid_sample where the
+    coordinates are finite."""
+    import ctypes
+    import math
+    from rsna_knee_efficiency_amd import hip
+    n, sk = 11, 5
+    print(f"grid forms kind={kind} {h}x{w} view={view}", flush=True)
+    g = torch.Generator().manual_seed(h * w)
+    if view == "noise":
+        grid = (torch.rand((h, w, 2), generator=g) * 2.4 - 1.2).half().to(dev)
+    else:
+        a = math.radians(20) if view == "turn" else 0.0
+        s = view if isinstance(view, float) else 1.1
+        theta = torch.tensor([[[math.cos(a) / s, -math.sin(a) / s, 0.03], [math.sin(a) / s, math.cos(a) / s, -0.02]]])
+        grid = F.affine_grid(theta, (1, 1, h, w), align_corners=False)[0].half().to(dev).contiguous()
+        if view == "nan":
+            pick = torch.rand((h, w), generator=g).to(dev)
+            grid[pick < 0.02] = float("nan")
+            grid[pick > 0.98] = float("inf")
+    lut = tta.lut_u8_f16(dev)
+    idx = torch.randint(0, sk, (n,), generator=g).to(dev)
+    if kind == 1:
+        src = torch.randint(0, 256, (sk, h, w), generator=g, dtype=torch.uint8).to(dev)
+        imgs = lut[src[idx].long()]
+    else:
+        src = torch.rand((n, h, w), generator=g).half().to(dev)
+        imgs = src
+    outs = []
+    for shift in (0, 1):                           # an output at an odd element takes the one-pixel form
+        buf = torch.full((8 + n * h * w + 8,), 9.0, dtype=torch.float16, device=dev)
+        a = hip.GridArgs(src=src.data_ptr(), slice_idx=idx.data_ptr(), lut=lut.data_ptr(), grid=grid.data_ptr(),
+                         out=buf.data_ptr() + 16 - 2 * shift, kind=kind, N=n, H=h, W=w, B=1, SK=sk, M=n)
+        hip.call("d8s_grid_sample", ctypes.byref(a), ctypes.c_void_p(torch.cuda.current_stream(dev).cuda_stream))
+        assert bool((buf[:8 - shift] == 9).all()) and bool((buf[n * h * w + 8 - shift:] == 9).all())
+        outs.append(buf[8 - shift:8 - shift + n * h * w].view(n, h, w).clone())
+    assert torch.equal(outs[0].view(torch.int16), outs[1].view(torch.int16))
+    if view != "nan":
+        want = F.grid_sample(imgs[:, None], grid.expand(n, h, w, 2), mode="bilinear", padding_mode="zeros",
+                             align_corners=False)[:, 0]
+        assert torch.equal(outs[0], want)
