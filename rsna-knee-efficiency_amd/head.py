@@ -49,12 +49,13 @@ class KneeHead:
         self.heads = int(context_heads)
         if self.CD != 64 * self.heads:
             raise ValueError(f"context width {self.CD} with {self.heads} heads: 64 per head is required")
-        self._ws: torch.Tensor | None = None
-        # the last slot_of_window seen (kept alive, so identity and version name its contents) and
-        # its checked int32 copy on the device: a fixed window layout is validated once, not per call
-        self._slot_src: torch.Tensor | None = None
-        self._slot_ver = -1
-        self._slot_dev: torch.Tensor | None = None
+        # workspaces per stream: calls on two streams at once do not share one
+        self._ws = hip.StreamBuffers()
+        # the last slot_of_window seen (kept alive, so identity and version name its contents), its
+        # version and its checked int32 copy on the device: a fixed window layout is validated once,
+        # not per call.  One tuple, replaced whole (another thread may be reading it)
+        self._slots_seen: tuple | None = None
+        self._in_graphs: list = []             # copies that captured calls read
 
     def _args(self, z, slot_of, mask, logits) -> hip.HeadArgs:
         a = hip.HeadArgs()
@@ -69,16 +70,18 @@ class KneeHead:
     def _slots(self, slot_of_window: torch.Tensor) -> torch.Tensor:
         """slot_of_window as int32 on the device, checked to lie in 0 .. S-1 (the reference's embedding
         lookup raises on such an index).  The check reads the values on the host, so it runs once per
-        tensor and in-place version: later calls with the same unchanged tensor reuse the checked copy."""
-        if (self._slot_src is slot_of_window and slot_of_window._version == self._slot_ver
-                and self._slot_dev is not None):
-            return self._slot_dev
+        tensor and in-place version: later calls with the same unchanged tensor reuse the checked copy
+        (complete when it is made: a copy from host memory waits)"""
+        seen = self._slots_seen
+        if seen is not None and seen[0] is slot_of_window and seen[1] == slot_of_window._version:
+            return seen[2]
+        version = slot_of_window._version
         host = slot_of_window.detach().to("cpu", torch.int64).reshape(-1)
         if bool(((host < 0) | (host >= self.S)).any()):
             raise ValueError("slot_of_window outside 0 .. S-1")
-        self._slot_dev = host.to(torch.int32).to(self.device)
-        self._slot_src, self._slot_ver = slot_of_window, slot_of_window._version
-        return self._slot_dev
+        on_device = host.to(torch.int32).to(self.device)
+        self._slots_seen = (slot_of_window, version, on_device)
+        return on_device
 
     def __call__(self, encoded: torch.Tensor, slot_of_window: torch.Tensor, slot_mask: torch.Tensor,
                  window_index: torch.Tensor | None = None) -> torch.Tensor:
@@ -97,12 +100,16 @@ class KneeHead:
         a = self._args(z, slot_of, mask, logits)
         need = ctypes.c_uint64()
         hip.call("d8s_head_workspace", ctypes.byref(a), ctypes.byref(need))
-        if self._ws is None or self._ws.numel() < need.value + 256:
-            self._ws = torch.empty(int(need.value) + 256, dtype=torch.uint8, device=self.device)
-        base = (self._ws.data_ptr() + 255) // 256 * 256
-        a.workspace, a.ws_bytes = base, self._ws.numel() - (base - self._ws.data_ptr())
-        stream = torch.cuda.current_stream(self.device).cuda_stream
-        hip.call("d8s_head", ctypes.byref(a), ctypes.c_void_p(stream))
+        stream = torch.cuda.current_stream(self.device)
+        slot_of.record_stream(stream)          # (another thread's call may replace the kept copy)
+        if hip.capturing(stream) and not any(t is slot_of for t in self._in_graphs):
+            self._in_graphs.append(slot_of)
+        bufs = self._ws.of(stream)
+        with bufs.lock:
+            ws = bufs.get("ws", int(need.value) + 256, self.device)
+            base = (ws.data_ptr() + 255) // 256 * 256
+            a.workspace, a.ws_bytes = base, ws.numel() - (base - ws.data_ptr())
+            hip.call("d8s_head", ctypes.byref(a), ctypes.c_void_p(stream.cuda_stream))
         return logits
 
 

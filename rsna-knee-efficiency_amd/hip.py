@@ -12,6 +12,7 @@ There is no fallback: if the library is missing, `library()` raises.
 """
 from __future__ import annotations
 
+import collections
 import ctypes
 import hashlib
 import threading
@@ -279,3 +280,54 @@ def written(*tensors) -> None:
     for t in tensors:
         if t is not None:
             torch.autograd.graph.increment_version(t)
+
+
+class BufferSet:
+    """Named device buffers of one stream's calls, grown on demand; hold `lock` from asking for them until
+    the launches that use them are enqueued (another thread may be on the same stream)."""
+
+    def __init__(self) -> None:
+        self.lock = threading.Lock()
+        self._mem: dict[str, torch.Tensor] = {}
+
+    def get(self, name: str, nbytes: int, device) -> torch.Tensor:
+        t = self._mem.get(name)
+        if t is None or t.numel() < nbytes:
+            t = self._mem[name] = torch.empty(int(nbytes), dtype=torch.uint8, device=device)
+        return t
+
+
+class StreamBuffers:
+    """Work buffers that are kept between calls: one `BufferSet` per stream, so calls on different streams
+    share no memory, and calls on one stream follow each other on it.  Each set is allocated with its
+    stream current, so the allocator orders its release, too, after that stream's work.  The sets of the
+    last `limit` streams are kept; a call on a capturing stream gets a set of its own, which lies in the
+    graph's memory and is not kept."""
+
+    def __init__(self, limit: int = 4) -> None:
+        self.limit = limit
+        self._lock = threading.Lock()
+        self._sets: collections.OrderedDict = collections.OrderedDict()
+
+    def of(self, stream: torch.cuda.Stream) -> BufferSet:
+        """The set of `stream`, which is the current one of its device."""
+        if capturing(stream):
+            return BufferSet()
+        key = (stream.device_index, stream.cuda_stream)
+        with self._lock:
+            found = self._sets.get(key)
+            if found is None:
+                found = self._sets[key] = BufferSet()
+                if len(self._sets) > self.limit:
+                    self._sets.popitem(last=False)
+            else:
+                self._sets.move_to_end(key)
+            return found
+
+
+def capturing(stream: torch.cuda.Stream) -> bool:
+    """Whether `stream` is being captured into a graph."""
+    if torch.cuda.current_device() == stream.device_index and torch.cuda.current_stream() == stream:
+        return torch.cuda.is_current_stream_capturing()
+    with torch.cuda.stream(stream):
+        return torch.cuda.is_current_stream_capturing()

@@ -140,3 +140,62 @@ def test_head_product_and_fusion_edges(dev, d, w, cd, targets, b):
     got = head.KneeHead(sd, dev, context_heads=cd // 64)(z.to(dev), slot_of, mask).cpu()
     scale = want.abs().max().item()
     assert (got - want).abs().max().item() <= 4e-6 * max(scale, 1.0)
+
+
+def test_head_on_two_streams_and_threads(dev):
+    """One head called from two streams at once, then from two threads on one stream and on two, with layouts
+    of their own: every call's logits are those of the call alone."""
+    import threading
+    sd = H.random_state_dict(31)
+    hd = head.KneeHead(sd, dev)
+    cases = []
+    for b, w, seed in ((8, 88, 1), (6, 66, 2)):
+        z, slot_of, mask = _case(b, w, seed)
+        z, mask = z.to(dev), mask.to(dev)
+        cases.append((z, slot_of, mask, hd(z, slot_of, mask).clone()))
+    torch.cuda.synchronize(dev)
+
+    def calls(case, stream, out, n=40):
+        z, slot_of, mask, _ = case
+        with torch.cuda.stream(stream):
+            for _ in range(n):
+                out.append(hd(z, slot_of, mask))
+
+    streams = [torch.cuda.Stream(dev) for _ in range(2)]
+    got = [[], []]
+    for _ in range(40):                              # one thread, the two streams in turn
+        for k in range(2):
+            calls(cases[k], streams[k], got[k], 1)
+    for pair in (streams, [streams[0]] * 2):         # two threads
+        ts = [threading.Thread(target=calls, args=(cases[k], pair[k], got[k])) for k in range(2)]
+        for t in ts:
+            t.start()
+        for t in ts:
+            t.join()
+    torch.cuda.synchronize(dev)
+    for k in range(2):
+        assert len(got[k]) == 120
+        for g in got[k]:
+            assert torch.equal(g, cases[k][3])
+
+
+def test_head_captured_call_keeps_its_layout(dev):
+    """A captured call's replays, after the head has seen another layout and larger calls: the captured layout's
+    logits."""
+    sd = H.random_state_dict(32)
+    hd = head.KneeHead(sd, dev)
+    z, slot_of, mask = _case(2, 44, 3)
+    z, mask = z.to(dev), mask.to(dev)
+    want = hd(z, slot_of, mask).clone()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        out = hd(z, slot_of, mask)
+    z2, slot2, mask2 = _case(8, 88, 4)
+    for k in range(3):
+        slot2 = slot2.flip(0).clone()
+        hd(z2.to(dev), slot2, mask2)
+        fill = [torch.full((44,), 7, dtype=torch.int32, device=dev) for _ in range(64)]
+        g.replay()
+        torch.cuda.synchronize(dev)
+        assert torch.equal(out, want), k
+        del fill

@@ -264,3 +264,24 @@ def test_recorded_kernel_variants(plan169):
     names = [set(t.values()) for t in (dense8s.C1_VARIANTS, dense8s.C2_VARIANTS, dense8s.TRANS_VARIANTS)]
     assert all(len(n) == len(t) for n, t in zip(names, (dense8s.C1_VARIANTS, dense8s.C2_VARIANTS,
                                                         dense8s.TRANS_VARIANTS)))
+
+
+def test_stream_buffers_are_per_stream(monkeypatch):
+    """Work buffers: one set per stream, grown on demand, the longest unused given up past the limit; a
+    capturing stream's call gets a set that is not kept."""
+    import types
+    busy = []
+    monkeypatch.setattr(hip, "capturing", lambda s: s in busy)
+    a, b, c = (types.SimpleNamespace(device_index=0, cuda_stream=k) for k in (1, 2, 3))
+    bufs = hip.StreamBuffers(limit=2)
+    sa = bufs.of(a)
+    ta = sa.get("ws", 100, "cpu")
+    assert bufs.of(a) is sa and sa.get("ws", 50, "cpu") is ta and ta.numel() == 100
+    assert sa.get("ws", 200, "cpu").numel() == 200 and sa.get("other", 10, "cpu").numel() == 10
+    sb = bufs.of(b)
+    assert sb is not sa and sb.get("ws", 100, "cpu").data_ptr() != sa.get("ws", 100, "cpu").data_ptr()
+    bufs.of(a)
+    bufs.of(c)                                       # b is the longest unused
+    assert bufs.of(a) is sa and bufs.of(b) is not sb
+    busy.append(a)
+    assert bufs.of(a) is not sa and bufs.of(a) is not bufs.of(a)
