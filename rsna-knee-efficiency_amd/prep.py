@@ -77,19 +77,16 @@ def read_range(k_sl: int, flip: int, read_slices: tuple[int, int] | None) -> tup
     return (k_sl - z, k_sl - a) if flip == FLIP_SLICES else (a, z)
 
 
+# The workspace and the float32 scratch of d8s_prep calls, a set per stream (calls on two streams at once
+# share nothing), and per device the workspace of the latest call (its head holds that call's stats)
+_BUFFERS = hip.StreamBuffers()
 _WS: dict = {}
 
 
-def _workspace(device: torch.device, n: int, img: int) -> torch.Tensor:
-    """Device workspace for d8s_prep (kept per device and grown on demand)."""
+def _workspace_bytes(n: int, img: int) -> int:
     need = ctypes.c_uint64()
     hip.call("d8s_prep_workspace", n, img, ctypes.byref(need))
-    key = str(device)
-    ws = _WS.get(key)
-    if ws is None or ws.numel() < need.value:
-        ws = torch.empty(int(need.value) + 256, dtype=torch.uint8, device=device)
-        _WS[key] = ws
-    return ws
+    return int(need.value)
 
 
 def _aligned_ptr(ws: torch.Tensor) -> int:
@@ -97,40 +94,28 @@ def _aligned_ptr(ws: torch.Tensor) -> int:
     return (p + 255) // 256 * 256
 
 
-_SCRATCH: dict = {}
-
-
-def _scratch(device: torch.device, nbytes: int) -> torch.Tensor:
-    """Device scratch for the resized float32 stacks of a kind-0 d8s_prep call (kept per device and
-    grown on demand)."""
-    key = str(device)
-    sc = _SCRATCH.get(key)
-    if sc is None or sc.numel() * 4 < nbytes:
-        sc = torch.empty((nbytes + 3) // 4, dtype=torch.float32, device=device)
-        _SCRATCH[key] = sc
-    return sc
-
-
 def _run(entry: str, kind: int, img: int, stacks: list[dict], device: torch.device) -> torch.Tensor:
     """Launches `entry` over `stacks` (dicts of D8sPrepStack fields), 16 at a time, on the current
-    stream.  Returns the workspace (its head holds the stats of the last chunk).  Calls on one device
-    share the workspace and scratch: they are ordered by the stream they are issued on."""
-    ws = _workspace(device, hip.PREP_MAX_STACKS, img)
-    stream = torch.cuda.current_stream(device).cuda_stream
-    for c in range(0, len(stacks), hip.PREP_MAX_STACKS):
-        chunk = stacks[c:c + hip.PREP_MAX_STACKS]
-        a = hip.PrepArgs()
-        a.workspace = _aligned_ptr(ws)
-        a.ws_bytes = ws.numel() - (a.workspace - ws.data_ptr())
-        if entry == "d8s_prep" and kind == 0:
-            need = sum(4 * (s["k1"] - s["k0"]) * img * img for s in chunk)
-            sc = _scratch(device, need)
-            a.scratch, a.scratch_bytes = sc.data_ptr(), sc.numel() * 4
-        a.kind, a.img, a.n_stacks = kind, img, len(chunk)
-        for i, s in enumerate(chunk):
-            for k, v in s.items():
-                setattr(a.s[i], k, v)
-        hip.call(entry, ctypes.byref(a), ctypes.c_void_p(stream))
+    stream.  Returns the workspace (its head holds the stats of the last chunk).  Calls on one stream
+    share the workspace and scratch: they follow each other on it."""
+    stream = torch.cuda.current_stream(device)
+    bufs = _BUFFERS.of(stream)
+    with bufs.lock:
+        ws = bufs.get("ws", _workspace_bytes(hip.PREP_MAX_STACKS, img) + 256, device)
+        for c in range(0, len(stacks), hip.PREP_MAX_STACKS):
+            chunk = stacks[c:c + hip.PREP_MAX_STACKS]
+            a = hip.PrepArgs()
+            a.workspace = _aligned_ptr(ws)
+            a.ws_bytes = ws.numel() - (a.workspace - ws.data_ptr())
+            if entry == "d8s_prep" and kind == 0:
+                sc = bufs.get("scratch", sum(4 * (s["k1"] - s["k0"]) * img * img for s in chunk), device)
+                a.scratch, a.scratch_bytes = sc.data_ptr(), sc.numel()
+            a.kind, a.img, a.n_stacks = kind, img, len(chunk)
+            for i, s in enumerate(chunk):
+                for k, v in s.items():
+                    setattr(a.s[i], k, v)
+            hip.call(entry, ctypes.byref(a), ctypes.c_void_p(stream.cuda_stream))
+        _WS[str(device)] = ws
     return ws
 
 

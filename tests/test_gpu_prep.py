@@ -216,3 +216,46 @@ def test_float_levels_counts(dev, r, k, img, kind):
     got = hp.to_uint8_hist_batch(torch.from_numpy(x).to(dev)).cpu().numpy()
     for i in range(r):
         assert np.array_equal(got[i], P.to_uint8(x[i])), i
+
+
+def test_prep_on_two_streams_and_threads(dev):
+    """Preparations of different studies and float stacks from two streams at once, then from two threads on
+    two streams and on one: every call's bytes are those of the call alone."""
+    import threading
+    img, K = 128, 8
+    spec = hp.PrepSpec(img=img, slices=K, n_seq=4, n_scales=2)
+    jobs = []
+    for b in range(2):
+        pay = synthetic.study_payload(img, K, 40 + b, series=_series(True))
+        pay = dict(pay, raw=torch.as_tensor(pay["raw"]).to(dev), u8=torch.as_tensor(pay["u8"]).to(dev))
+        x = torch.rand((3, 4, 96, 96), generator=torch.Generator().manual_seed(b)).to(dev) * (b + 1)
+        jobs.append((pay, x))
+
+    def one(job):
+        pay, x = job
+        return hp.payloads_to_uint8([pay], spec, dev), hp.to_uint8_hist_batch(x)
+
+    want = [one(j) for j in jobs]
+    torch.cuda.synchronize(dev)
+
+    def calls(k, stream, out, n=15):
+        with torch.cuda.stream(stream):
+            for _ in range(n):
+                out.append(one(jobs[k]))
+
+    streams = [torch.cuda.Stream(dev) for _ in range(2)]
+    got = [[], []]
+    for _ in range(15):
+        for k in range(2):
+            calls(k, streams[k], got[k], 1)
+    for pair in (streams, [streams[0]] * 2):
+        ts = [threading.Thread(target=calls, args=(k, pair[k], got[k])) for k in range(2)]
+        for t in ts:
+            t.start()
+        for t in ts:
+            t.join()
+    torch.cuda.synchronize(dev)
+    for k in range(2):
+        assert len(got[k]) == 45
+        for vol, u8 in got[k]:
+            assert torch.equal(vol, want[k][0]) and torch.equal(u8, want[k][1])
