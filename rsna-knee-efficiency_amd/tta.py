@@ -25,25 +25,35 @@ _GRIDS: dict = {}
 _LUTS: dict = {}
 
 
+def _kept(book: dict, key, make, device) -> torch.Tensor:
+    """book[key], made on first use.  The first use waits for it, so that any stream may read it from then on;
+    under capture it belongs to the graph, which makes it again at every replay, and is not kept."""
+    t = book.get(key)
+    if t is None:
+        t = make()
+        if torch.device(device).type == "cuda":
+            stream = torch.cuda.current_stream(device)
+            if hip.capturing(stream):
+                return t
+            stream.synchronize()
+        t = book.setdefault(key, t)
+    return t
+
+
 def lut_u8_f16(device) -> torch.Tensor:
     """fp16 u / 255 for u = 0..255 as the reference builds it (fused_uint8.py:735)."""
-    key = str(device)
-    if key not in _LUTS:
-        _LUTS[key] = torch.arange(256, dtype=torch.uint8, device=device).half().mul_(1.0 / 255.0)
-    return _LUTS[key]
+    return _kept(_LUTS, str(device),
+                 lambda: torch.arange(256, dtype=torch.uint8, device=device).half().mul_(1.0 / 255.0), device)
 
 
 def view_grid(h: int, w: int, d: int, scale: float, tx: float, ty: float, dtype, device) -> torch.Tensor:
     """The (H, W, 2) grid of the view: `F.affine_grid` of theta [[1/s, 0, -2 tx], [0, 1/s, -2 ty]]
     (src/knee/tta.py:141-146)."""
-    key = (h, w, d, float(scale), float(tx), float(ty), dtype, str(device))
-    g = _GRIDS.get(key)
-    if g is None:
+    def make():
         theta = torch.tensor([[1.0 / scale, 0.0, -2.0 * tx], [0.0, 1.0 / scale, -2.0 * ty]],
                              device=device, dtype=dtype).unsqueeze(0)
-        g = F.affine_grid(theta, (1, d, h, w), align_corners=False)[0].contiguous()
-        _GRIDS[key] = g
-    return g
+        return F.affine_grid(theta, (1, d, h, w), align_corners=False)[0].contiguous()
+    return _kept(_GRIDS, (h, w, d, float(scale), float(tx), float(ty), dtype, str(device)), make, device)
 
 
 def _sample(args: hip.GridArgs, device) -> None:
@@ -100,11 +110,11 @@ def windows_u8(v_u8: torch.Tensor, slice_idx: torch.Tensor, out: torch.Tensor, s
         raise ValueError("out must be a contiguous fp16 tensor of B * len(slice_idx) images")
     idx = slice_idx.contiguous()
     _check_slices(idx, s * k)
-    gp = 0
-    if not (scale == 1.0 and tx == 0.0 and ty == 0.0):
-        gp = view_grid(h, w, 1, scale, tx, ty, torch.float16, v_u8.device).data_ptr()
-    a = hip.GridArgs(src=v_u8.data_ptr(), slice_idx=idx.data_ptr(), lut=lut_u8_f16(v_u8.device).data_ptr(),
-                     grid=gp, out=out.data_ptr(), kind=1, N=b * m, H=h, W=w, B=b, SK=s * k, M=m)
+    identity = scale == 1.0 and tx == 0.0 and ty == 0.0
+    grid = None if identity else view_grid(h, w, 1, scale, tx, ty, torch.float16, v_u8.device)
+    lut = lut_u8_f16(v_u8.device)
+    a = hip.GridArgs(src=v_u8.data_ptr(), slice_idx=idx.data_ptr(), lut=lut.data_ptr(),
+                     grid=0 if grid is None else grid.data_ptr(), out=out.data_ptr(), kind=1, N=b * m, H=h, W=w, B=b, SK=s * k, M=m)
     _sample(a, v_u8.device)
     hip.written(out)
     return out

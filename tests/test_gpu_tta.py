@@ -272,3 +272,28 @@ def test_grid_sample_forms(dev, kind, h, w, view):
         want = F.grid_sample(imgs[:, None], grid.expand(n, h, w, 2), mode="bilinear", padding_mode="zeros",
                              align_corners=False)[:, 0]
         assert torch.equal(outs[0], want)
+
+
+def test_view_grid_made_on_a_busy_stream(dev):
+    """A view's grid is made on the stream that first asks for it; a second stream that asks while the first is
+    still busy gets the finished grid."""
+    h, w = 48, 64
+    g = torch.Generator().manual_seed(8)
+    v = torch.randint(0, 256, (1, 2, 4, h, w), generator=g, dtype=torch.uint8).to(dev)
+    idx = torch.tensor([0, 1, 2, 5, 6, 7], dtype=torch.int64, device=dev)
+    tta.windows_u8(v, idx, torch.empty((2, 3, h, w), dtype=torch.float16, device=dev))    # (idx checked)
+    lut = tta.lut_u8_f16(dev)
+    x = lut[v.view(1, 8, h, w).index_select(1, idx).long()].view(1, 2, 3, h, w)
+    torch.cuda.synchronize(dev)
+    for scale in (1.1375, 0.8625):
+        outs = [torch.zeros((2, 3, h, w), dtype=torch.float16, device=dev) for _ in range(2)]
+        torch.cuda.synchronize(dev)
+        streams = [torch.cuda.Stream(dev) for _ in range(2)]
+        with torch.cuda.stream(streams[0]):
+            torch.cuda._sleep(50_000_000)
+            tta.windows_u8(v, idx, outs[0], scale)
+        with torch.cuda.stream(streams[1]):
+            tta.windows_u8(v, idx, outs[1], scale)
+        torch.cuda.synchronize(dev)
+        want = _reference(x, scale, 0.0, 0.0).view(2, 3, h, w)
+        assert torch.equal(outs[0], want) and torch.equal(outs[1], want)
