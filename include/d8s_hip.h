@@ -452,7 +452,7 @@ int d8s_head(const D8sHeadArgs* a, void* stream);
  * for callers that cannot allocate device memory (code under HIP graph capture, tight serving loops,
  * harnesses that forbid hipMalloc).  Same arguments and results as d8s_head; a->workspace and
  * a->ws_bytes are ignored.  The workspace is a static device array of D8S_HEAD_SCRATCH_BYTES per GPU
- * (32 MiB: up to 28 studies of 128 windows, or 41 of 88, at the final configuration), held until the
+ * (32 MiB: up to 31 studies of 128 windows, or 45 of 88, at the final configuration), held until the
  * process ends; a call whose d8s_head_workspace() exceeds it is rejected with hipErrorInvalidValue.
  * `stream` must belong to the current device.  Every call on a GPU uses that GPU's one array, so calls
  * that overlap on one GPU (unordered streams) race: order them on one stream or with events. */

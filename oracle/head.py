@@ -25,7 +25,8 @@ def head_forward(sd: dict, encoded: torch.Tensor, slot_of: torch.Tensor, slot_ma
     cd = sd["ctx_in.weight"].shape[0]
     pos = torch.arange(w) % per
     h = f @ sd["ctx_in.weight"].t() + sd["ctx_in.bias"] + sd["ctx_pos"][pos].unsqueeze(0)
-    layer = nn.TransformerEncoderLayer(cd, heads, dim_feedforward=2 * cd, dropout=0.0, batch_first=True,
+    ff = sd["ctx.layers.0.linear1.weight"].shape[0]
+    layer = nn.TransformerEncoderLayer(cd, heads, dim_feedforward=ff, dropout=0.0, batch_first=True,
                                        norm_first=True)
     enc = nn.TransformerEncoder(layer, 1, enable_nested_tensor=False)
     enc.load_state_dict({k[len("ctx."):]: v for k, v in sd.items() if k.startswith("ctx.layers.")})
@@ -45,7 +46,8 @@ def head_forward(sd: dict, encoded: torch.Tensor, slot_of: torch.Tensor, slot_ma
 
 
 def random_state_dict(seed: int, d: int = 1664, slots: int = 8, per: int = 11, cd: int = 256,
-                      targets: int = 12) -> dict:
+                      targets: int = 12, ff: int | None = None) -> dict:
+    ff = 2 * cd if ff is None else ff
     g = torch.Generator().manual_seed(seed)
 
     def r(*shape, s=0.02):
@@ -57,8 +59,8 @@ def random_state_dict(seed: int, d: int = 1664, slots: int = 8, per: int = 11, c
           "ctx.layers.0.self_attn.in_proj_bias": r(3 * cd),
           "ctx.layers.0.self_attn.out_proj.weight": r(cd, cd, s=1 / cd ** 0.5),
           "ctx.layers.0.self_attn.out_proj.bias": r(cd),
-          "ctx.layers.0.linear1.weight": r(2 * cd, cd, s=1 / cd ** 0.5), "ctx.layers.0.linear1.bias": r(2 * cd),
-          "ctx.layers.0.linear2.weight": r(cd, 2 * cd, s=1 / (2 * cd) ** 0.5),
+          "ctx.layers.0.linear1.weight": r(ff, cd, s=1 / cd ** 0.5), "ctx.layers.0.linear1.bias": r(ff),
+          "ctx.layers.0.linear2.weight": r(cd, ff, s=1 / ff ** 0.5),
           "ctx.layers.0.linear2.bias": r(cd),
           "ctx.layers.0.norm1.weight": 1 + r(cd, s=0.1), "ctx.layers.0.norm1.bias": r(cd),
           "ctx.layers.0.norm2.weight": 1 + r(cd, s=0.1), "ctx.layers.0.norm2.bias": r(cd),

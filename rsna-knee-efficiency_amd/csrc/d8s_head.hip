@@ -808,6 +808,13 @@ struct Ws {
     uint64_t bytes;
 };
 
+// The workspace: what lives from launch 2 to the end, and two regions used in turn by what does not.
+//   region 1: launch 1's raw sums (read by 2), qkv (3 to 4), the partial dots (5 to 6);
+//   region 2: LN1(h) (2 to 3) and Mo's raw sums (1 to 2), which become Mo in float64 in place (k_head_rows adds
+//             the splits' sums of an element and writes it in one thread; read by 3); then what launch 4, or 4
+//             and the out_proj product, leave for 5.
+// So a call takes no more than one that kept every intermediate of the unfolded head (at most 8192 wide, 65536
+// hidden units), whatever the K split.
 Ws carve(const D8sHeadArgs* a, char* base) {
     Ws w{};
     const uint64_t M = (uint64_t)a->B * a->W, T2 = 2ull * a->T;
@@ -819,30 +826,33 @@ Ws carve(const D8sHeadArgs* a, char* base) {
     };
     const Split sp = split_plan((int64_t)M, a->CD + (int)T2, a->D);
     w.h = take(M * a->CD);
-    w.qkv = take(3 * M * a->CD);
     w.d0 = take(M * T2);
     w.mo = take(T2 * a->CD);
-    w.mod = (double*)take(2 * T2 * a->CD);
     w.mf = take(T2 * a->FF);
     w.dc = take(T2);
-    w.part = take((uint64_t)((a->FF + FS - 1) / FS) * M * T2);
     w.valid = (uint8_t*)take((M + 3) / 4);
-    // the raw sums of launch 1 (read by launch 2), and in their place what launches 4 and 5 exchange;
-    // LN1(h) (launches 2 and 3) likewise before it
-    const uint64_t o0 = off;
-    w.hn = take(M * a->CD);
+    uint64_t o0 = off, end = off;
+    auto region = [&]() { off = o0; };
+    auto done = [&]() { end = std::max(end, off); };
     w.cs = take((uint64_t)sp.splits * M * (a->CD + T2));
+    done(), region();
+    w.qkv = take(3 * M * a->CD);
+    done(), region();
+    w.part = take((uint64_t)((a->FF + FS - 1) / FS) * M * T2);
+    done();
+    o0 = off = end;
+    w.hn = take(M * a->CD);
     w.ms = (double*)take(2 * (uint64_t)sp.splits * T2 * a->CD);
-    const uint64_t o1 = off;
-    off = o0;
+    w.mod = w.ms;
+    done(), region();
     if (fuse_out(a)) {
         w.hp = take((uint64_t)a->heads * M * a->CD);
     } else {
         w.att = take(M * a->CD);
         w.h1 = take(M * a->CD);
     }
-    off = std::max(off, o1);
-    w.bytes = off;
+    done();
+    w.bytes = end;
     return w;
 }
 

@@ -321,3 +321,45 @@ def test_conv2_choice_by_tiles(n, h, w, variant):
     lib = hip.library()
     a = hip.Conv2Args(0x1000, 0x1000, 0x1000, 0x1000, 0x1000, n, h, w, 0)
     assert lib.d8s_conv2_variant(ctypes.byref(a), 0) == variant
+
+
+def test_head_scratch_holds_what_the_unfolded_head_needed():
+    """`d8s_head_noalloc` takes every call whose intermediates, each in a buffer of its own (h, qkv, the
+    attention, h1, the hidden units, h2, the dots of every 64 features), and whose K split's sums fit its
+    scratch, up to 128 heads; and the study counts its documentation names, no more."""
+    scratch = 32 << 20
+    lib = hip.library()
+    need = ctypes.c_uint64()
+
+    def bytes_of(b, w, d, cd, t, ff):
+        a = _head_args(B=b, W=w, D=d, CD=cd, heads=cd // 64, FF=ff, T=t)
+        assert lib.d8s_head_workspace(ctypes.byref(a), ctypes.byref(need)) == 0
+        return need.value
+
+    def unfolded(b, w, d, cd, t, ff):
+        m = b * w
+        sums = 0
+        for n, k in ((cd, d), (3 * cd, cd), (cd, cd), (ff, cd), (cd, ff)):
+            chunks, tiles = -(-k // 64), -(-m // 64) * -(-n // 64)
+            if tiles < 256 and chunks > 1:
+                per = -(-chunks // min(chunks, -(-512 // tiles)))
+                sums = max(sums, 4 * -(-chunks // per) * m * n)
+        return 4 * m * (7 * cd + ff + 2 * t * (-(-d // 64) + 1)) + sums
+
+    tried = 0
+    for d in (1, 130, 602, 1664, 4096):
+        for cd in (64, 192, 256, 320, 512, 2048, 4096, 8192):
+            for t in (1, 12, 16):
+                for ff in (1, 8, 72, 2 * cd, 65536):
+                    for w in (1, 8, 88, 128):
+                        lo, hi = 0, 65535
+                        while lo < hi:
+                            b = (lo + hi + 1) // 2
+                            lo, hi = (b, hi) if unfolded(b, w, d, cd, t, ff) <= scratch else (lo, b - 1)
+                        for b in {lo, lo * 9 // 10, lo // 2, 1} if lo else ():
+                            if b and b * w * d < 2 ** 31:
+                                tried += 1
+                                assert bytes_of(b, w, d, cd, t, ff) <= scratch, (b, w, d, cd, t, ff)
+    assert tried > 5000
+    for b, w in ((31, 128), (45, 88)):
+        assert bytes_of(b, w, 1664, 256, 12, 512) <= scratch < bytes_of(b + 1, w, 1664, 256, 12, 512)

@@ -78,3 +78,17 @@ def test_noalloc_rejects_sizes_beyond_the_scratch(dev):
         hip.call("d8s_head_noalloc", ctypes.byref(a), stream)
     torch.cuda.synchronize(dev)
     assert torch.equal(logits, torch.full_like(logits, 7.0))   # nothing ran
+
+
+def test_noalloc_small_heads_of_many_studies(dev):
+    """A call near the scratch's size whose K is split in two (2254 studies of one window, 8 heads, one hidden
+    unit): the workspace entry's logits, and the oracle's."""
+    sd = H.random_state_dict(23, d=130, slots=3, per=4, cd=512, targets=16, ff=1)
+    hd = head.KneeHead(sd, dev, context_heads=8)
+    g = torch.Generator().manual_seed(23)
+    z = torch.randn((2254, 1, 130), generator=g) * 0.5
+    slot_of, mask = torch.tensor([1]), torch.rand((2254, 3), generator=g) < 0.8
+    want, got, need = _both(hd, z, slot_of, mask, dev)
+    assert need <= SCRATCH_BYTES
+    assert torch.equal(got, want)
+    assert torch.allclose(got, H.head_forward(sd, z, slot_of, mask, heads=8), rtol=1e-4, atol=1e-4)
