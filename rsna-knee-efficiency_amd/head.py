@@ -102,9 +102,9 @@ class KneeHead:
         hip.call("d8s_head_workspace", ctypes.byref(a), ctypes.byref(need))
         stream = torch.cuda.current_stream(self.device)
         slot_of.record_stream(stream)          # (another thread's call may replace the kept copy)
-        if hip.capturing(stream) and not any(t is slot_of for t in self._in_graphs):
-            self._in_graphs.append(slot_of)
         bufs = self._ws.of(stream)
+        if bufs.captured and not any(t is slot_of for t in self._in_graphs):
+            self._in_graphs.append(slot_of)
         with bufs.lock:
             ws = bufs.get("ws", int(need.value) + 256, self.device)
             base = (ws.data_ptr() + 255) // 256 * 256

@@ -286,8 +286,9 @@ class BufferSet:
     """Named device buffers of one stream's calls, grown on demand; hold `lock` from asking for them until
     the launches that use them are enqueued (another thread may be on the same stream)."""
 
-    def __init__(self) -> None:
+    def __init__(self, captured: bool = False) -> None:
         self.lock = threading.Lock()
+        self.captured = captured               # the call is being recorded into a graph
         self._mem: dict[str, torch.Tensor] = {}
 
     def get(self, name: str, nbytes: int, device) -> torch.Tensor:
@@ -312,7 +313,7 @@ class StreamBuffers:
     def of(self, stream: torch.cuda.Stream) -> BufferSet:
         """The set of `stream`, which is the current one of its device."""
         if capturing(stream):
-            return BufferSet()
+            return BufferSet(captured=True)
         key = (stream.device_index, stream.cuda_stream)
         with self._lock:
             found = self._sets.get(key)
@@ -326,8 +327,8 @@ class StreamBuffers:
 
 
 def capturing(stream: torch.cuda.Stream) -> bool:
-    """Whether `stream` is being captured into a graph."""
-    if torch.cuda.current_device() == stream.device_index and torch.cuda.current_stream() == stream:
+    """Whether `stream`, the current one of its device, is being captured into a graph."""
+    if torch.cuda.current_device() == stream.device_index:
         return torch.cuda.is_current_stream_capturing()
-    with torch.cuda.stream(stream):
+    with torch.cuda.device(stream.device_index):
         return torch.cuda.is_current_stream_capturing()
