@@ -703,7 +703,7 @@ def kind_us(b: dict, kind: str, n: int, cus: int = 256) -> float:
                      6 and 8 tiles at g = 23), whatever the count of bands that fit it, and the rows its
                      workgroups exchange (0.3 us per thousand pixels of them);
       img            14.4 us a round at g = 35;
-      chain          a launch of 8.6 us at g = 9 and 13 us per full round of three workgroups per CU;
+      chain          a launch of 10.4 us at g = 9, 8.6 and 13 per full round of three workgroups per CU;
       tile           rounds of 32 x 12 (narrower maps: 16 x 12) tiles, 3.8 + 13 us (3.8 + 7.7) at g = 9;
                      64 and 128 wide: rounds of row bands (`_band_steps`);
       conv           two launches, 12 us at g = 9 (16 beyond one round), and their bytes, conv2's with its
@@ -720,7 +720,7 @@ def kind_us(b: dict, kind: str, n: int, cus: int = 256) -> float:
     if name == "img":
         return -(-n // cus) * (5.2 + 0.26 * g)
     if name == "chain":
-        return 6.2 + 0.25 * g + 13.2 * kpx / (0.384 * cus)
+        return max(8.0 + 0.25 * g, 6.2 + 0.25 * g + 13.2 * kpx / (0.384 * cus))
     if name == "tile":
         if w in (64, 128) and block_groups(b) <= BAND_MAX_GROUPS:
             return 1.5 + 0.55 * g + (0.95 + 0.1 * g) * w / 64 * _band_steps(h, w, n, cus)
@@ -742,15 +742,26 @@ def _band_steps(h: int, w: int, n: int, cus: int) -> int:
 BAND_US = ((1, (5.9, 0.02)), (2, (7.0, 0.045)), (4, (8.6, 0.07)), (6, (10.0, 0.11)), (8, (11.6, 0.16)))
 
 
+# Default banded kinds have at most a CU count's `BAND_SHARE`-th of bands per image.  A banded launch that is
+# not wholly resident can hold one CU less than an image's bands without progress; launches of other
+# runners, ordered by nobody, progress only while such images leave a CU free: BAND_SHARE of them do.
+BAND_SHARE = 8
+
+
+def bounded_options(b: dict, n: int, cus: int = 256) -> list[str]:
+    """`kind_options` without the banded kinds of more than cus / `BAND_SHARE` bands per image."""
+    return [k for k in kind_options(b, n) if ":" not in k or int(k.split(":", 1)[1]) * BAND_SHARE <= cus]
+
+
 def default_kind(b: dict, n: int, cus: int = 256) -> str:
-    """The block kind of block `b` at n images per pass: the least `kind_us` of the kinds it can take
-    (ties to the earlier one).  A map of a whole workgroup's 256 pixels whose images make more than a
+    """The block kind of block `b` at n images per pass: the least `kind_us` of `bounded_options` (ties to
+    the earlier one).  A map that fits a workgroup per image and whose images make more than a
     quarter of the CUs stays "img" though two bands per image are faster alone: its one workgroup per
     image leaves room for a second encoder's pass on another stream, which 2-band launches did not
     (5.8 against 6.3-6.8 ms per study of two seeds at 96 images)."""
     if img_fits(b) and b["h"] * b["w"] == IMG_MAX_PX and cus < 4 * n <= 4 * cus:
         return "img"
-    return min(kind_options(b, n), key=lambda kind: kind_us(b, kind, n, cus))
+    return min(bounded_options(b, n, cus), key=lambda kind: kind_us(b, kind, n, cus))
 
 
 def valid_kind(b: dict, bi: int, kind, n: int, cus: int = 256) -> str:

@@ -145,9 +145,10 @@ def odd_maps(dev):
         model = densenet.seeded_densenet169(6, blocks=(2, 2, 4, 3)).to(dev)
         x_u8 = synthetic.study_u8(n, img, seed=4)
         cal = dense8s.calibrate(model, [synthetic.normalise(torch.from_numpy(x_u8).to(dev))])
-        pack = dense8s.make_pack(dense8s.make_plan(model.cpu(), cal, img), n, input_kind="u8")
+        plan = dense8s.make_plan(model.cpu(), cal, img)
+        pack = dense8s.make_pack(plan, n, input_kind="u8")
         x = torch.from_numpy(x_u8).to(dev)
-        out[img] = {"pack": pack, "x": x, "n": n,
+        out[img] = {"plan": plan, "pack": pack, "x": x, "n": n,
                     "want": dense8s.Dense8SEncoder(pack, dev.index or 0, n, fused={})(x).clone()}
     return out
 
@@ -173,6 +174,31 @@ def test_bands_same_bytes(dev, odd_maps, img, block, bands):
         torch.cuda.synchronize(dev)
         assert torch.equal(g, m["want"])
     assert enc.sync_errors() == 0
+
+
+def test_bands_unordered_runners(dev, odd_maps):
+    """Four one-image runners with default kinds, each called from a stream of its own with nothing between
+    them: every pass's features, and no wait runs out."""
+    img = 288
+    plan = odd_maps[img]["plan"]
+    pack = dense8s.make_pack(plan, 1, input_kind="u8")
+    encs = [dense8s.Dense8SEncoder(pack, dev.index or 0, 1) for _ in range(4)]
+    assert encs[0].max_bands > 1
+    print(f"unordered runners, kinds {encs[0].fused}", flush=True)
+    xs = [odd_maps[img]["x"][k % 3:k % 3 + 1].contiguous() for k in range(4)]
+    want = [odd_maps[img]["want"][k % 3:k % 3 + 1] for k in range(4)]
+    for e in encs:
+        e.capture(1)
+    streams = [torch.cuda.Stream(dev) for _ in encs]
+    torch.cuda.synchronize(dev)
+    for rep in range(20):
+        for e, x, st in zip(encs, xs, streams):
+            with torch.cuda.stream(st):
+                e(x)
+    torch.cuda.synchronize(dev)
+    for e, w in zip(encs, want):
+        assert torch.equal(e.out[:1], w)
+    assert sum(e.sync_errors() for e in encs) == 0
 
 
 def test_parts_wait_error_surfaces(dev, c4):

@@ -285,3 +285,26 @@ def test_stream_buffers_are_per_stream(monkeypatch):
     assert bufs.of(a) is sa and bufs.of(b) is not sb
     busy.append(a)
     assert bufs.of(a) is not sa and bufs.of(a) is not bufs.of(a)
+
+
+def _blocks(img: int) -> list:
+    out, c = [], 64
+    for i, layers in enumerate((6, 12, 32, 32)):
+        out.append(dict(h=img // 4 >> i, w=img // 4 >> i, c0=c, L=layers, trans=i < 3))
+        c = (c + 32 * layers) // 2
+    return out
+
+
+def test_default_kinds_leave_room_for_unordered_runners():
+    """Eight passes with default kinds, ordered by nobody, always make progress: each may hold one CU less than
+    an image's bands, and together they leave one free.  Kinds a caller names are not bounded."""
+    for cus in (256, 64):
+        for img in range(96, 513, 32):
+            for n in (1, 2, 3, 4, 8, 24, 96):
+                for bi, b in enumerate(_blocks(img)):
+                    kind = dense8s.default_kind(b, n, cus)
+                    bands = int(kind.split(":")[1]) if ":" in kind else 1
+                    assert dense8s.BAND_SHARE * (bands - 1) < cus, (img, n, kind)
+                    assert dense8s.valid_kind(b, bi, kind, n, cus) == kind
+    b = _blocks(288)[0]
+    assert dense8s.valid_kind(b, 0, "bands:72", 1) == "bands:72"
