@@ -753,13 +753,23 @@ def bounded_options(b: dict, n: int, cus: int = 256) -> list[str]:
     return [k for k in kind_options(b, n) if ":" not in k or int(k.split(":", 1)[1]) * BAND_SHARE <= cus]
 
 
+TWO_BANDS_PX = 100              # see default_kind
+
+
 def default_kind(b: dict, n: int, cus: int = 256) -> str:
     """The block kind of block `b` at n images per pass: the least `kind_us` of `bounded_options` (ties to
-    the earlier one).  A map that fits a workgroup per image and whose images make more than a
-    quarter of the CUs stays "img" though two bands per image are faster alone: its one workgroup per
-    image leaves room for a second encoder's pass on another stream, which 2-band launches did not
-    (5.8 against 6.3-6.8 ms per study of two seeds at 96 images)."""
-    if img_fits(b) and b["h"] * b["w"] == IMG_MAX_PX and cus < 4 * n <= 4 * cus:
+    the earlier one).  A map that fits a workgroup per image stays "img" where the images make more than
+    a quarter of the CUs and half of the map is more than `TWO_BANDS_PX` pixels: two bands of four whole
+    pixel tiles are faster alone, but hold twice the CUs for 0.8 of the time and are slower beside a
+    second encoder's pass.  ms of one pass alone and of two seeds at once (`encode_concurrent`), 96
+    images, block 3 as "img" and as two bands:
+        512 px (16 x 16, 128 pixels a band)  3.10 / 3.02   5.81 / 5.96
+        480 px (15 x 15, 120)                3.28 / 3.21   5.99 / 6.17
+        448 px (14 x 14, 98)                 3.04 / 2.97   6.17 / 6.06
+        416 px (13 x 13, 91)                 2.85 / 2.78   5.08 / 5.12
+        288 px (9 x 9, 45)                   1.77 / 1.63   2.84 / 2.67
+    (at 72 images the same: 480 px 4.82 / 5.00, 416 px 3.89 / 3.76)."""
+    if img_fits(b) and -(-b["h"] // 2) * b["w"] > TWO_BANDS_PX and cus < 4 * n <= 4 * cus:
         return "img"
     return min(bounded_options(b, n, cus), key=lambda kind: kind_us(b, kind, n, cus))
 

@@ -295,6 +295,19 @@ def _blocks(img: int) -> list:
     return out
 
 
+def test_default_kind_of_large_batches():
+    """One workgroup per image by the map's size, not at one size: from bands of more than 100 pixels, at more
+    than a quarter of the CUs' images."""
+    kind = lambda h, w, n, cus=256: dense8s.default_kind(dict(h=h, w=w, c0=640, L=32), n, cus)  # noqa: E731
+    for h, w in ((16, 16), (15, 15), (8, 32), (15, 16), (12, 20)):
+        for n in (65, 72, 96, 128):
+            assert kind(h, w, n) == "img", (h, w, n)
+        assert kind(h, w, 48) != "img"
+    for h, w in ((14, 14), (13, 13), (9, 9)):
+        assert kind(h, w, 96) == "bands:2", (h, w)
+    assert kind(15, 15, 24, 64) == "img"
+
+
 def test_default_kinds_leave_room_for_unordered_runners():
     """Eight passes with default kinds, ordered by nobody, always make progress: each may hold one CU less than
     an image's bands, and together they leave one free.  Kinds a caller names are not bounded."""
