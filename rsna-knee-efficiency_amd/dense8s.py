@@ -1160,7 +1160,11 @@ class Dense8SEncoder(_PassRunner):
         self.library_version = hip.version()
         self.pack_sha = meta.get("kernels_sha")
         self.nb = int(meta["n"])
-        self.fused = fused_blocks(meta, fused, _cu_count(self.dev))
+        cus = _cu_count(self.dev)
+        self.fused = fused_blocks(meta, fused, cus)
+        # the blocks whose kind neither the caller nor the package chose
+        self.default_blocks = frozenset(bi for bi, b in enumerate(meta["blocks"])
+                                        if fused is None and recorded_kind(b, bi, self.nb, cus) is None)
         self.variants = recorded_variants(meta)  # {(family, block[, layer]): kernel variant}
         self.n_out = -(-int(n_total) // self.nb) * self.nb
         self.max_inflight = max_inflight
@@ -1315,15 +1319,23 @@ class Dense8SEncoder(_PassRunner):
         return steps
 
     def _compile(self) -> None:
-        """The program of one pass: the stem, each block's layers as its kind, its transition, and the
-        final features (the launch sequence of the reference's `_pass`, `src/knee/dense8s.py:1354-1385`)."""
+        """The runner's own program: `build` of its kinds."""
+        self.program = self.build(self.fused)
+        # bands per image of the widest banded launch: its share of the CUs a wait needs resident
+        self.max_bands = widest_bands(self.program)
+        self._checked = self.max_bands > 0
+
+    def build(self, kinds: dict) -> list[Step]:
+        """The program of one pass with the given kind per block: the stem, each block's layers, its
+        transition, and the final features (the launch sequence of the reference's `_pass`,
+        `src/knee/dense8s.py:1354-1385`)."""
         img = int(self.meta["img"])
-        self.stem_args = hip.StemArgs(0, _ptr(self.par["S_lut"]), _ptr(self.par["S_w16"]),
+        stem_args = hip.StemArgs(0, _ptr(self.par["S_lut"]), _ptr(self.par["S_w16"]),
                                       _ptr(self.par["S_bias"]), _ptr(self.par["S_inv"]), self.in0[0],
                                       self.nb, img, img, self.in_kind, 0, 0)
-        prog = [Step("stem", 0, -1, ((0, 0),), "d8s_stem", self.stem_args)]
+        prog = [Step("stem", 0, -1, ((0, 0),), "d8s_stem", stem_args)]
         for bi, b in enumerate(self.meta["blocks"]):
-            prog += self.block_steps(bi, self.fused[bi])
+            prog += self.block_steps(bi, kinds[bi])
             if b["trans"]:
                 g0, hw = b["c0"] // GROUP, b["h"] * b["w"]
                 cout = (b["c0"] + GROWTH * b["L"]) // 2
@@ -1342,17 +1354,16 @@ class Dense8SEncoder(_PassRunner):
                     raise ValueError(f"{step.label()}: kernel variant {VARIANTS[step.family][v]!r} is not "
                                      f"taken for this shape")
                 step.variant = v
-        self.program = prog
-        self._checked = any(s.entry in BANDED_ENTRIES for s in prog)
-        # bands per image of the widest banded launch: its share of the CUs a wait needs resident
-        self.max_bands = max((s.args.parts for s in prog if s.entry in BANDED_ENTRIES), default=0)
-        if self._checked and self._report is None:
+        if widest_bands(prog):
+            prog[-1].entry = "d8s_final_checked"
+        if widest_bands(prog) and self._report is None:
             # a host-mapped word the final kernel copies the banded blocks' error count into
             self._report = torch.zeros(2, dtype=torch.int32).pin_memory()
             self._report_np = self._report.numpy()
             dptr = ctypes.c_void_p()
             hip.check(self.lib.d8s_host_mapped(self._report.data_ptr(), ctypes.byref(dptr)), "d8s_host_mapped")
             self._report_dev = int(dptr.value or 0)
+        return prog
 
     def _variant_of(self, step: Step) -> int:
         """The kernel variant `variants` gives a conv1, conv2 or transition launch (0: none)."""
@@ -1373,7 +1384,7 @@ class Dense8SEncoder(_PassRunner):
             b = self.meta["blocks"][step.block]
             common = (self.in0[step.block], b["c0"] // GROUP, self.seg[step.block], self.nb,
                       b["h"] * b["w"], _ptr(self.par["F_ab"]), f_ptr, self.meta["n_features"])
-            if self._checked:
+            if step.entry == "d8s_final_checked":
                 rc = lib.d8s_final_checked(*common, _ptr(self._sync) + 8, self._report_dev, st)
             else:
                 rc = lib.d8s_final(*common, st)
@@ -1660,6 +1671,7 @@ class Dense8SEncoder(_PassRunner):
         if apply:
             self.fused = {bi: min(out[f"b{bi}"].items(), key=lambda kv: kv[1])[0]
                           for bi in range(len(self.meta["blocks"]))}
+            self.default_blocks = frozenset()
             self.graphs.clear()
             self._compile()
         return out
@@ -1779,9 +1791,32 @@ def concurrent_order(runners, cus: int = 256) -> list[list[int]]:
     return order
 
 
+def widest_bands(program: list[Step]) -> int:
+    """Bands per image of the widest banded launch of a program (0: none)."""
+    return max((s.args.parts for s in program if s.entry in BANDED_ENTRIES), default=0)
+
+
 PAIR_ENTRIES = {"d8s_stem": "d8s_stem_pair", "d8s_conv1": "d8s_conv1_pair", "d8s_conv2": "d8s_conv2_pair",
                 "d8s_dense": "d8s_dense_pair", "d8s_dense_block": "d8s_dense_block_pair",
                 "d8s_transition": "d8s_transition_pair"}
+
+
+PAIRED_KINDS = ("conv", "tile", "img")     # the block kinds whose launches carry both encoders
+
+
+def pair_kind(b: dict, n: int, cus: int = 256) -> str:
+    """The kind of block `b` (meta) for two encoders of n images in one sequence.  From n past an eighth of
+    the CUs the least time of both, `kind_us` of 2 n images where one launch carries both and twice that of
+    n where it does not; below, where the per-layer launches hardly overlap, `default_kind`.  Two seeds, ms,
+    with the kinds a runner defaults to alone and with the least time of both:
+        96 images  288 px 3.13 / 2.95  416 px 5.45 / 4.75  480 px 6.08 / 5.87  512 px 5.52 / 5.47
+        48 images  288 px 2.12 / 2.12  416 px 3.25 / 2.89  480 px 3.65 / 3.46  512 px 3.50 / 3.24
+        24 images  288 px 1.68 / 2.38  416 px 2.22 / 2.18  480 px 2.47 / 2.35  512 px 2.31 / 2.23
+         8 images  288 px 1.37 / 1.53  416 px 1.53 / 1.66  480 px 1.73 / 2.32  512 px 1.50 / 1.87"""
+    if 8 * n <= cus:
+        return default_kind(b, n, cus)
+    return min(bounded_options(b, n, cus),
+               key=lambda k: kind_us(b, k, 2 * n, cus) if k in PAIRED_KINDS else 2 * kind_us(b, k, n, cus))
 
 
 class EncoderPair(_PassRunner):
@@ -1790,7 +1825,8 @@ class EncoderPair(_PassRunner):
     entry point (`PAIR_ENTRIES`, `d8s_*_pair`) one launch carrying both encoders' arguments, so the two
     passes' small late layers fill the chip together (the 16 x 16 whole block: 192 workgroups in about
     the time of 96) instead of overlapping by chance on two streams (`encode_concurrent`); the other
-    steps (banded blocks, chained launches, final features) as two launches in the same sequence.  Each
+    steps (banded blocks, chained launches, final features) as two launches in the same sequence.  Blocks
+    whose kind both encoders left to the default run as `pair_kind`, the others as the encoders' own.  Each
     encoder's outputs are exactly what it gives alone.  The pair launches on the first encoder's stream
     and orders the second's around it."""
 
@@ -1813,6 +1849,22 @@ class EncoderPair(_PassRunner):
         self.calls = {"graph": 0, "plain": 0, "copy": 0}
         self._gate = InflightGate(None)
         self._staging: torch.Tensor | None = None
+        self._built: tuple = ()
+
+    def programs(self) -> tuple[list[Step], list[Step]]:
+        """Both encoders' programs as the pair runs them, built again when a runner's own has changed."""
+        A, B = self.a, self.b
+        if not self._built or self._built[0] is not A.program or self._built[1] is not B.program:
+            kinds = dict(A.fused)
+            for bi in A.default_blocks & B.default_blocks:
+                kinds[bi] = pair_kind(A.meta["blocks"][bi], A.nb, _cu_count(self.dev))
+            progs = (A.program, B.program) if kinds == A.fused else (A.build(kinds), B.build(kinds))
+            self._built = (A.program, B.program, *progs)
+        return self._built[2:]
+
+    @property
+    def max_bands(self) -> int:
+        return max(widest_bands(p) for p in self.programs())
 
     def _owners(self) -> tuple:
         return (self.a, self.b)
@@ -1824,7 +1876,7 @@ class EncoderPair(_PassRunner):
     def _launch_pass(self, x_ptr: int, index: int, mode: int) -> None:
         A, B, st = self.a, self.b, self.stream.cuda_stream
         fa, fb = A.out[index * A.nb].data_ptr(), B.out[index * B.nb].data_ptr()
-        for sa, sb in zip(A.program, B.program):
+        for sa, sb in zip(*self.programs()):
             paired = None if sa.variant or sb.variant else PAIR_ENTRIES.get(sa.entry)
             if paired is None:
                 A._launch(sa, st, x_ptr, fa, mode)

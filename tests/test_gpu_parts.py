@@ -176,6 +176,33 @@ def test_bands_same_bytes(dev, odd_maps, img, block, bands):
     assert enc.sync_errors() == 0
 
 
+def test_pair_with_kinds_of_its_own(dev, odd_maps):
+    """A pair whose blocks run as other kinds than each encoder's own: each encoder's features, eager and
+    replayed; kinds the caller gave stay."""
+    m = odd_maps[416]
+    n = 65
+    pack = dense8s.make_pack(m["plan"], n, input_kind="u8")
+    encs = [dense8s.Dense8SEncoder(pack, dev.index or 0, n) for _ in range(2)]
+    x = m["x"][torch.arange(n, device=dev) % m["n"]].contiguous()
+    want = m["want"][torch.arange(n, device=dev) % m["n"]]
+    pair = dense8s.EncoderPair(*encs)
+    ran = [s.entry for s in pair.programs()[0]]
+    print(f"pair of {encs[0].fused}: {sorted(set(ran))}", flush=True)
+    assert ran != [s.entry for s in encs[0].program] and encs[0].max_bands > 0
+    for rep in range(3):
+        if rep == 1:
+            pair.capture(n)
+        fa, fb = pair(x)
+        assert torch.equal(fa, want) and torch.equal(fb, want), rep
+        assert torch.equal(encs[0](x), want)          # its own program beside the pair's
+    given = [dense8s.Dense8SEncoder(pack, dev.index or 0, n, fused=encs[0].fused) for _ in range(2)]
+    own = dense8s.EncoderPair(*given)
+    assert own.programs()[0] is given[0].program and own.max_bands == given[0].max_bands
+    fa, fb = own(x)
+    assert torch.equal(fa, want) and torch.equal(fb, want)
+    assert sum(e.sync_errors() for e in encs + given) == 0
+
+
 def test_bands_unordered_runners(dev, odd_maps):
     """Four one-image runners with default kinds, each called from a stream of its own with nothing between
     them: every pass's features, and no wait runs out."""

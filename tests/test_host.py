@@ -308,6 +308,17 @@ def test_default_kind_of_large_batches():
     assert kind(15, 15, 24, 64) == "img"
 
 
+def test_pair_kinds():
+    """A pair's kinds: one launch for both encoders' blocks where that is the least time of both, the runners'
+    own at small batches."""
+    for img, n, want in ((416, 96, ["conv", "conv", "conv", "img"]), (480, 96, ["conv", "conv", "conv", "img"]),
+                         (288, 96, ["conv", "conv", "bands:2", "img"]), (512, 48, ["tile", "conv", "conv", "img"])):
+        assert [dense8s.pair_kind(b, n) for b in _blocks(img)] == want, (img, n)
+    for img in (128, 288, 416, 512):
+        for b in _blocks(img):
+            assert dense8s.pair_kind(b, 24) == dense8s.default_kind(b, 24)
+
+
 def test_default_kinds_leave_room_for_unordered_runners():
     """Eight passes with default kinds, ordered by nobody, always make progress: each may hold one CU less than
     an image's bands, and together they leave one free.  Kinds a caller names are not bounded."""
