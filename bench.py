@@ -455,10 +455,20 @@ def _dispatch_counters(d: str) -> dict:
             name = r.get("Kernel_Name", "")
             if not _family(name):
                 continue
-            key = (name.split("(")[0].replace("void ", ""), r.get("Dispatch_Id", r.get("Correlation_Id", "")))
+            key = (name.split("(")[0].replace("void ", "").replace(", false>", ">"), r.get("Dispatch_Id", r.get("Correlation_Id", "")))
             c = out.setdefault(key, {})
             c[r["Counter_Name"]] = c.get(r["Counter_Name"], 0.0) + float(r["Counter_Value"])
     return out
+
+
+def _banded_kernel(b: dict, kind: str) -> str:
+    """The kernel of block `b` run as a banded kind, by its pixel tiles per band: `k_dparts<T>` of equal
+    bands of whole tiles ("parts"), `k_dparts<T, true>` of any other ("bands")."""
+    name, k = kind.split(":")
+    tiles = -(-(-(-b["h"] // int(k)) * b["w"]) // 32)
+    if name == "parts":
+        return f"k_dparts<{tiles}>"
+    return f"k_dparts<{tiles if tiles <= 2 else -(-tiles // 2) * 2}, true>"
 
 
 def c4_counter_summary(fetch_dir: str, write_dir: str, mfma_dir: str, wave_dir: str, passes: int,
@@ -487,9 +497,8 @@ def c4_counter_summary(fetch_dir: str, write_dir: str, mfma_dir: str, wave_dir: 
     kinds = dense8s.fused_blocks({"blocks": C5_BLOCKS, "n": n})
     work = {}
     for bi, b in enumerate(C5_BLOCKS):
-        if str(kinds[bi]).startswith("parts:"):
-            pt = b["h"] // int(kinds[bi].split(":")[1]) * b["w"] // 32
-            work[f"k_dparts<{pt}>"] = (bi, kinds[bi]) + block_work(b, n)
+        if ":" in kinds[bi]:
+            work[_banded_kernel(b, kinds[bi])] = (bi, kinds[bi]) + block_work(b, n)
     lines = [f"Calibration: k_copy moves {copy_bytes} B read + {copy_bytes} B written per dispatch; "
              f"FETCH_SIZE scale {kf:.3f}, WRITE_SIZE scale {kw:.3f}.", "",
              "| kernel | block (kind) | launches | HBM read MB | HBM write MB | traffic / algorithmic "

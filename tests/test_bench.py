@@ -236,6 +236,23 @@ def test_c4_counter_summary_per_banded_kernel(tmp_path):
     assert any(ln.startswith("| `k_dparts<1>`") for ln in out.splitlines())
 
 
+def test_c4_counter_summary_reads_todays_kernel_names(tmp_path):
+    """The banded kernels by the names a trace gives them: the equal bands' second template argument is
+    dropped, the ragged ones' kept."""
+    gib = 1 << 30
+    copy, k4 = "k_copy(const u32x4*, u32x4*, long)", "void k_dparts<4, false>(D8sPartsArgs)"
+    for name, ctr, scale in (("f", "FETCH_SIZE", 2), ("w", "WRITE_SIZE", 1)):
+        _counter_csv(tmp_path / name / "run_counter_collection.csv",
+                     [(1, copy, ctr, gib / scale / 1024), (2, k4, ctr, 10e6 / 1024)])
+    for name in "ms":
+        _counter_csv(tmp_path / name / "run_counter_collection.csv", [(2, k4, "GRBM_GUI_ACTIVE", 100.0)])
+    out = bench.c4_counter_summary(*(str(tmp_path / d) for d in "fwms"), passes=1)
+    assert any(ln.startswith("| `k_dparts<4>` | 2 (parts:8) | 1 | 20.00 | 10.00 |") for ln in out.splitlines()), out
+    assert bench._banded_kernel(dict(h=32, w=32), "parts:8") == "k_dparts<4>"
+    for h, w, k, want in ((18, 18, 18, 1), (36, 36, 36, 2), (9, 9, 1, 4), (36, 36, 9, 6), (36, 36, 6, 8)):
+        assert bench._banded_kernel(dict(h=h, w=w), f"bands:{k}") == f"k_dparts<{want}, true>"
+
+
 def test_family_roofline_divides_per_launch():
     # 31 launches of 100.8 MB in 0.837 ms per pass: 27 us per launch, 3.733 TB/s; 1 POP per pass
     fam, byts, ops = {"chain": 0.837}, {"chain": [100.8e6] * 31}, {"chain": 1e15 * 0.837e-3}
