@@ -5,8 +5,9 @@
 // Per study (W windows of D-dim encoder features, a few hundred KB) the head is a few small matrix
 // products with row-wise normalisations around them: latency, not arithmetic, is its cost (a call of 8
 // studies is 13 us of float32 MFMA work at peak).  So the work is arranged for few dependent launches
-// (six for all studies of a call), float32 throughout.  The logits use the context's output only
-// through its dots with attn.weight and cls_w (the 2T rows V of D values), so with
+// (six for all studies of a call), in float32; the small products Mo and Mf below are summed in float64.
+// The logits use the context's output only through its dots with attn.weight and cls_w (the 2T rows V of D
+// values), so with
 //   Mo = V ctx_out (2T x CD),  Mf = Mo ff2 (2T x FF)
 // every window's dots are V (z + slot_emb) + Mo h1 + Mf u + const, and neither the ff2 and ctx_out
 // products over the windows nor the features f2 are formed (55 % of the multiplications before):

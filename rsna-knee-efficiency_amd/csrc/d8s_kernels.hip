@@ -2666,7 +2666,6 @@ __global__ __launch_bounds__(DP_NT, 1) void k_dparts(D8sPartsArgs a) {
 #undef DP_LP
 #undef DP_G
 #undef DP_XP
-#undef DP_LDA
 #undef DP_GRP
 #undef DP_OFF
 #undef DP_RSRC

@@ -1308,18 +1308,16 @@ __global__ void __launch_bounds__(NT, KIND == 1 ? 7 : 4) k_grid_sample4(D8sGridA
 #define PREQ(cond, msg) \
     do { if (!(cond)) return d8s_host_fail((int)hipErrorInvalidValue, std::string(what) + ": " + (msg)); } while (0)
 
-// The workgroup ranges of every stack in the three grids (4 blocks per workgroup); returns the size of
-// the per-block grid.
+// The workgroup ranges of every stack in the grids of regions and of the final pass (4 blocks per workgroup;
+// the float32 levels' are wide_view's); returns the size of the per-block grid.
 int assign_grids(PArgs& a) {
-    int wh = 0, wh2 = 0, wn = 0;
+    int wh = 0, wn = 0;
     for (int i = 0; i < a.n; ++i) {
         PStack& p = a.s[i];
-        p.hb = p.hb2 = p.nb = 4;
+        p.hb = p.nb = 4;
         p.wg_hist = wh;
-        p.wg_hist2 = wh2;
         p.wg_norm = wn;
         wh += (p.nblk + p.hb - 1) / p.hb;
-        wh2 += (p.nblk + p.hb2 - 1) / p.hb2;
         wn += (p.nblk + p.nb - 1) / p.nb;
     }
     return wn;
@@ -1344,8 +1342,8 @@ PArgs float_view(const PArgs& a) {
 }
 
 // The view the wide workgroups read: float32 stacks in blocks of about 16384 pixels (four 16-byte loads a
-// thread of a wide workgroup), as many blocks a workgroup as leave about four workgroups a CU (a study's
-// level 3 takes 38 us so, 44 with two a CU).
+// thread of a wide workgroup), as many blocks a workgroup as make a grid of about four workgroups per CU, two
+// of them resident at a time (a study's level 3 takes 38 us so, 44 with a grid of two per CU).
 PArgs wide_view(const PArgs& a) {
     PArgs f = a;
     const int rb = a.img >= 16384 ? 1 : 16384 / a.img;
