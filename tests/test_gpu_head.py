@@ -142,6 +142,28 @@ def test_head_product_and_fusion_edges(dev, d, w, cd, targets, b):
     assert (got - want).abs().max().item() <= 4e-6 * max(scale, 1.0)
 
 
+@pytest.mark.parametrize("d,w,cd,ff,b", [
+    (96, 20, 256, 200, 2),           # a partial slice of hidden units and column tile, four heads unfused
+    (64, 5, 64, 1, 3),               # one hidden unit
+    (130, 33, 128, 72, 1),           # a slice of 8 units, two heads fused
+    (64, 17, 256, 512, 1),           # 4 x 256 = 2 x 256 + 512: the last feed-forward width that fuses four heads
+    (64, 17, 256, 511, 1),           # and the first that does not
+])
+def test_head_feed_forward_widths(dev, d, w, cd, ff, b):
+    """Feed-forward widths that are no multiple of a slice, and both sides of the rule that fuses out_proj into
+    the attention, against the float32 oracle: within 4e-6 of the largest logit (at most 512 products a sum,
+    about 32 roundings of 2^-24, twice that for the fold's own sums)."""
+    sd = H.random_state_dict(d + ff, d=d, slots=4, per=5, cd=cd, targets=12, ff=ff)
+    g = torch.Generator().manual_seed(ff)
+    z = torch.randn((b, w, d), generator=g) * 0.5
+    slot_of = torch.arange(w) % 4
+    mask = torch.rand((b, 4), generator=g) > 0.3
+    mask[0] = True
+    want = H.head_forward(sd, z, slot_of, mask, heads=cd // 64)
+    got = head.KneeHead(sd, dev, context_heads=cd // 64)(z.to(dev), slot_of, mask).cpu()
+    assert (got - want).abs().max().item() <= 4e-6 * max(want.abs().max().item(), 1.0)
+
+
 def test_head_on_two_streams_and_threads(dev):
     """One head called from two streams at once, then from two threads on one stream and on two, with layouts
     of their own: every call's logits are those of the call alone."""

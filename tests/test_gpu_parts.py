@@ -176,6 +176,31 @@ def test_bands_same_bytes(dev, odd_maps, img, block, bands):
     assert enc.sync_errors() == 0
 
 
+@pytest.mark.parametrize("img,n,kinds", [
+    (288, 64, {1: "bands:8", 2: "bands:3", 3: "bands:3"}),       # 512 and 192 workgroups; 36, 18 and 9 wide
+    (416, 65, {2: "bands:5", 3: "bands:4"}),                      # 325 and 260: bands of 6 and 5, 4 and 3 rows
+])
+def test_bands_several_rounds_and_two_runners(dev, odd_maps, img, n, kinds):
+    """Ragged bands of more workgroups than CUs (an image's bands start as others end), alone and with a second
+    runner's ragged bands beside them (`encode_concurrent`), eager and replayed."""
+    m = odd_maps[img]
+    print(f"bands in rounds img={img} n={n} {kinds}", flush=True)
+    pack = dense8s.make_pack(m["plan"], n, input_kind="u8")
+    encs = [dense8s.Dense8SEncoder(pack, dev.index or 0, n, fused=kinds) for _ in range(2)]
+    pick = torch.arange(n, device=dev) % m["n"]
+    x, want = m["x"][pick].contiguous(), m["want"][pick]
+    xs, wants = [x, x.flip(0).contiguous()], [want, want.flip(0)]
+    for rep in range(3):
+        if rep == 1:
+            for e in encs:
+                e.capture(n)
+        assert torch.equal(encs[0](x), want), rep
+        outs = [o.clone() for o in dense8s.encode_concurrent([(e, v, False) for e, v in zip(encs, xs)])]
+        torch.cuda.synchronize(dev)
+        assert all(torch.equal(o, w) for o, w in zip(outs, wants)), rep
+    assert sum(e.sync_errors() for e in encs) == 0
+
+
 def test_pair_with_kinds_of_its_own(dev, odd_maps):
     """A pair whose blocks run as other kinds than each encoder's own: each encoder's features, eager and
     replayed; kinds the caller gave stay."""

@@ -130,10 +130,11 @@ def test_windows_u8_slice_checks(dev, view):
     assert torch.equal(out2, ref)
 
 
-@pytest.mark.parametrize("kind", [0, 1])
+SHIFTED_VIEWS = [(1.5, 0.0, 0.0), (1.25, 0.11, -0.2), (0.8, 0.0, 0.05), (0.6, 0.0, 0.0), (1.0, 0.02, 0.0)]
+
+
+@pytest.mark.parametrize("kind,view", [(1, (1.0, 0.0, 0.0))] + [(k, v) for k in (0, 1) for v in SHIFTED_VIEWS])
 @pytest.mark.parametrize("h,w,off", [(5, 4, 0), (7, 8, 0), (9, 12, 0), (33, 64, 0), (33, 64, 1), (20, 61, 0), (3, 3, 1)])
-@pytest.mark.parametrize("view", [(1.0, 0.0, 0.0), (1.5, 0.0, 0.0), (1.25, 0.11, -0.2), (0.8, 0.0, 0.05), (0.6, 0.0, 0.0),
-                                  (1.0, 0.02, 0.0)])
 def test_grid_sample_kernels_agree(dev, kind, h, w, off, view):
     """The four-pixel form's three paths (zoom in, zoom out, borders), narrow and odd images, images that
     start at an odd element (`off`: the one-pixel form, the gather's unaligned loads) and group remainders,
@@ -141,8 +142,6 @@ def test_grid_sample_kernels_agree(dev, kind, h, w, off, view):
     values, and nothing written around the output."""
     import ctypes
     from rsna_knee_efficiency_amd import hip
-    if kind == 0 and view == (1.0, 0.0, 0.0):
-        pytest.skip("fp16 images have no gather")
     n, sk = 19, 5
     print(f"grid kind={kind} {h}x{w} off={off} view={view}", flush=True)
     g = torch.Generator().manual_seed(h * w + off)
