@@ -707,7 +707,10 @@ def kind_us(b: dict, kind: str, n: int, cus: int = 256) -> float:
       tile           rounds of 32 x 12 (narrower maps: 16 x 12) tiles, 3.8 + 13 us (3.8 + 7.7) at g = 9;
                      64 and 128 wide: rounds of row bands (`_band_steps`);
       conv           two launches, 12 us at g = 9 (16 beyond one round), and their bytes, conv2's with its
-                     32 x 8 tiles' padding."""
+                     32 x 8 tiles' padding.
+    Over 120 (side, batch) pairs of that range the four blocks run as the kinds of least estimate take 1.2 %
+    more than as the fastest ones on average, 14 % at most (bands of several rounds, estimated up to 50 %
+    high where the rounds overlap)."""
     h, w, g = b["h"], b["w"], b["c0"] / GROUP + (b["L"] - 1) / 2
     kpx = n * h * w / 1000
     name = _kind_name(kind)

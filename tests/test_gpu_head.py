@@ -101,13 +101,13 @@ def test_head_abi_slot_outside_range_reads_nothing(dev):
 
 
 @pytest.mark.parametrize("d,w,slots,per,cd,targets,b", [
-    (602, 37, 5, 7, 128, 5, 3),      # depth not a multiple of 4 (scalar weight staging), odd windows
+    (602, 37, 5, 7, 128, 5, 3),      # depth not a multiple of 4, odd windows
     (640, 16, 2, 16, 192, 16, 1),    # 3 heads, 16 findings, one query group
     (100, 129 - 1, 8, 11, 64, 1, 2),  # one head, one finding, 128 windows, a partial column tile
 ])
 def test_head_other_shapes(dev, d, w, slots, per, cd, targets, b):
-    """Shapes away from the final configuration: partial product tiles in every dimension, the
-    scalar weight path, 1-3 heads, 1-16 findings, other slot and position counts."""
+    """Shapes away from the final configuration: partial product tiles in every dimension, 1-3 heads,
+    1-16 findings, other slot and position counts."""
     sd = H.random_state_dict(d + w, d=d, slots=slots, per=per, cd=cd, targets=targets)
     g = torch.Generator().manual_seed(w)
     z = torch.randn((b, w, d), generator=g) * 0.5

@@ -295,6 +295,15 @@ def _blocks(img: int) -> list:
     return out
 
 
+def test_default_kinds_at_the_documented_sizes():
+    for img, n, want in ((512, 24, ["tile", "chain", "parts:8", "parts:8"]), (512, 96, ["tile", "conv", "chain", "img"]),
+                         (288, 88, ["conv", "conv", "bands:2", "bands:2"]),
+                         (288, 11, ["tile", "bands:12", "bands:18", "bands:3"]),
+                         (416, 37, ["conv", "conv", "bands:4", "bands:4"]),
+                         (512, 1, ["conv", "parts:32", "parts:32", "parts:8"])):
+        assert [dense8s.default_kind(b, n) for b in _blocks(img)] == want, (img, n)
+
+
 def test_default_kind_of_large_batches():
     """One workgroup per image by the map's size, not at one size: from bands of more than 100 pixels, at more
     than a quarter of the CUs' images."""
