@@ -1324,6 +1324,7 @@ class Dense8SEncoder(_PassRunner):
     def _compile(self) -> None:
         """The runner's own program: `build` of its kinds."""
         self.program = self.build(self.fused)
+        self.stem_args = self.program[0].args
         # bands per image of the widest banded launch: its share of the CUs a wait needs resident
         self.max_bands = widest_bands(self.program)
         self._checked = self.max_bands > 0

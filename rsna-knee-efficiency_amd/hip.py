@@ -310,6 +310,9 @@ class StreamBuffers:
         self._lock = threading.Lock()
         self._sets: collections.OrderedDict = collections.OrderedDict()
 
+    def __reduce__(self):                      # a copy of an owner has buffers of its own
+        return StreamBuffers, (self.limit,)
+
     def of(self, stream: torch.cuda.Stream) -> BufferSet:
         """The set of `stream`, which is the current one of its device."""
         if capturing(stream):

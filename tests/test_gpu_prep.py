@@ -259,3 +259,21 @@ def test_prep_on_two_streams_and_threads(dev):
         assert len(got[k]) == 45
         for vol, u8 in got[k]:
             assert torch.equal(vol, want[k][0]) and torch.equal(u8, want[k][1])
+
+
+def test_captured_preparation_replays(dev):
+    """A captured `to_uint8_hist_batch` replayed between other preparations: its own bytes every time."""
+    g = torch.Generator().manual_seed(9)
+    xs = [torch.rand((2, 3, 96, 96), generator=g).to(dev) * (k + 1) for k in range(2)]
+    want = [hp.to_uint8_hist_batch(x).clone() for x in xs]
+    out = torch.zeros(xs[0].shape, dtype=torch.uint8, device=dev)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        hp.to_uint8_hist_batch(xs[0], out)
+    for rep in range(3):
+        out.zero_()
+        assert torch.equal(hp.to_uint8_hist_batch(xs[1]), want[1])
+        graph.replay()
+        assert torch.equal(hp.to_uint8_hist_batch(xs[1]), want[1])
+        torch.cuda.synchronize(dev)
+        assert torch.equal(out, want[0]), rep

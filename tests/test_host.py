@@ -285,6 +285,9 @@ def test_stream_buffers_are_per_stream(monkeypatch):
     assert bufs.of(a) is sa and bufs.of(b) is not sb
     busy.append(a)
     assert bufs.of(a) is not sa and bufs.of(a) is not bufs.of(a)
+    import copy
+    twin = copy.deepcopy(bufs)
+    assert twin.limit == 2 and twin.of(b) is not bufs.of(b)
 
 
 def _blocks(img: int) -> list:
