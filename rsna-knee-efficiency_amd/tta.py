@@ -25,35 +25,37 @@ _GRIDS: dict = {}
 _LUTS: dict = {}
 
 
-def _kept(book: dict, key, make, device) -> torch.Tensor:
-    """book[key], made on first use.  The first use waits for it, so that any stream may read it from then on;
-    under capture it belongs to the graph, which makes it again at every replay, and is not kept."""
-    t = book.get(key)
-    if t is None:
-        t = make()
-        if torch.device(device).type == "cuda":
-            stream = torch.cuda.current_stream(device)
-            if hip.capturing(stream):
-                return t
-            stream.synchronize()
-        t = book.setdefault(key, t)
-    return t
+def _keep(book: dict, key, t: torch.Tensor) -> torch.Tensor:
+    """Keeps `t`, just made on the current stream, as book[key], and waits for it, so that any stream may
+    read it from then on.  Made under capture it belongs to the graph, which makes it again at every
+    replay, and is not kept."""
+    if t.is_cuda:
+        stream = torch.cuda.current_stream(t.device)
+        if hip.capturing(stream):
+            return t
+        stream.synchronize()
+    return book.setdefault(key, t)
 
 
 def lut_u8_f16(device) -> torch.Tensor:
     """fp16 u / 255 for u = 0..255 as the reference builds it (fused_uint8.py:735)."""
-    return _kept(_LUTS, str(device),
-                 lambda: torch.arange(256, dtype=torch.uint8, device=device).half().mul_(1.0 / 255.0), device)
+    key = str(device)
+    lut = _LUTS.get(key)
+    if lut is None:
+        lut = _keep(_LUTS, key, torch.arange(256, dtype=torch.uint8, device=device).half().mul_(1.0 / 255.0))
+    return lut
 
 
 def view_grid(h: int, w: int, d: int, scale: float, tx: float, ty: float, dtype, device) -> torch.Tensor:
     """The (H, W, 2) grid of the view: `F.affine_grid` of theta [[1/s, 0, -2 tx], [0, 1/s, -2 ty]]
     (src/knee/tta.py:141-146)."""
-    def make():
+    key = (h, w, d, float(scale), float(tx), float(ty), dtype, str(device))
+    g = _GRIDS.get(key)
+    if g is None:
         theta = torch.tensor([[1.0 / scale, 0.0, -2.0 * tx], [0.0, 1.0 / scale, -2.0 * ty]],
                              device=device, dtype=dtype).unsqueeze(0)
-        return F.affine_grid(theta, (1, d, h, w), align_corners=False)[0].contiguous()
-    return _kept(_GRIDS, (h, w, d, float(scale), float(tx), float(ty), dtype, str(device)), make, device)
+        g = _keep(_GRIDS, key, F.affine_grid(theta, (1, d, h, w), align_corners=False)[0].contiguous())
+    return g
 
 
 def _sample(args: hip.GridArgs, device) -> None:
