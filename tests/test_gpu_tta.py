@@ -165,13 +165,13 @@ def test_grid_sample_kernels_agree(dev, kind, h, w, off, view):
     assert bool((out[:8] == 9).all()) and bool((out[-8:] == 9).all())
 
 
-@pytest.mark.parametrize("kind", [0, 1])
-def test_grid_sample_many_images(dev, kind):
+@pytest.mark.parametrize("kind,w,scale", [(0, 4, 1.1), (1, 4, 1.1), (0, 3, 1.1), (1, 3, 1.1), (1, 4, 1.0)])
+def test_grid_sample_many_images(dev, kind, w, scale):
     """As many images as the entry point takes (524287), past what one launch's y blocks of the four-pixel
-    form hold: every image as torch's grid_sample gives it."""
+    form hold, as the one-pixel form (3 wide) and as the gather: every image as torch's grid_sample gives it."""
     import ctypes
     from rsna_knee_efficiency_amd import hip
-    n, h, w, sk = 65536 * 8 - 1, 2, 4, 7
+    n, h, sk = 65536 * 8 - 1, 2, 7
     g = torch.Generator().manual_seed(3)
     lut = tta.lut_u8_f16(dev)
     idx = torch.randint(0, sk, (n,), generator=g).to(dev)
@@ -183,9 +183,13 @@ def test_grid_sample_many_images(dev, kind):
         imgs = src
     out = torch.full((n, h, w), 9.0, dtype=torch.float16, device=dev)
     grid = tta.view_grid(h, w, 1, 1.1, 0.0, 0.0, torch.float16, dev)
-    a = hip.GridArgs(src=src.data_ptr(), slice_idx=idx.data_ptr(), lut=lut.data_ptr(), grid=grid.data_ptr(),
-                     out=out.data_ptr(), kind=kind, N=n, H=h, W=w, B=1, SK=sk, M=n)
+    a = hip.GridArgs(src=src.data_ptr(), slice_idx=idx.data_ptr(), lut=lut.data_ptr(),
+                     grid=grid.data_ptr() if scale != 1.0 else 0, out=out.data_ptr(), kind=kind, N=n, H=h, W=w,
+                     B=1, SK=sk, M=n)
     hip.call("d8s_grid_sample", ctypes.byref(a), ctypes.c_void_p(torch.cuda.current_stream(dev).cuda_stream))
+    if scale == 1.0:
+        assert torch.equal(out, imgs[idx])
+        return
     # (torch's own launch over a batch of images; the volume's 7 slices once)
     want = torch.cat([F.grid_sample(c[:, None], grid.expand(len(c), h, w, 2), mode="bilinear", padding_mode="zeros",
                                     align_corners=False)[:, 0] for c in imgs.split(65536)])
