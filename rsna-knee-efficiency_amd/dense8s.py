@@ -1860,7 +1860,9 @@ class EncoderPair(_PassRunner):
         A, B = self.a, self.b
         if not self._built or self._built[0] is not A.program or self._built[1] is not B.program:
             kinds = dict(A.fused)
-            for bi in A.default_blocks & B.default_blocks:
+            # (kernel variants chosen for a block's launches keep its kind)
+            varied = {key[1] for e in (A, B) for key in e.variants if key[0] != "trans"}
+            for bi in (A.default_blocks & B.default_blocks) - varied:
                 kinds[bi] = pair_kind(A.meta["blocks"][bi], A.nb, _cu_count(self.dev))
             progs = (A.program, B.program) if kinds == A.fused else (A.build(kinds), B.build(kinds))
             self._built = (A.program, B.program, *progs)

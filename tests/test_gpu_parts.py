@@ -220,6 +220,12 @@ def test_pair_with_kinds_of_its_own(dev, odd_maps):
         fa, fb = pair(x)
         assert torch.equal(fa, want) and torch.equal(fb, want), rep
         assert torch.equal(encs[0](x), want)          # its own program beside the pair's
+    # block 1 (52 wide) runs fused alone and as two launches in the pair, unless a variant is recorded for it
+    entries = lambda prog, bi: {st.entry for st in prog if st.block == bi and st.family != "trans"}  # noqa: E731
+    assert entries(encs[0].program, 1) == {"d8s_dense"} and entries(pair.programs()[0], 1) == {"d8s_conv1", "d8s_conv2"}
+    varied = dict(pack, meta=dense8s.pack_meta(m["plan"], n, input_kind="u8", c2={52: "32x4"}))
+    kept = dense8s.EncoderPair(*(dense8s.Dense8SEncoder(varied, dev.index or 0, n) for _ in range(2)))
+    assert entries(kept.programs()[0], 1) == {"d8s_dense"}
     given = [dense8s.Dense8SEncoder(pack, dev.index or 0, n, fused=encs[0].fused) for _ in range(2)]
     own = dense8s.EncoderPair(*given)
     assert own.programs()[0] is given[0].program and own.max_bands == given[0].max_bands
